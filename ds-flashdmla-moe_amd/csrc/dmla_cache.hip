@@ -12,106 +12,141 @@
 namespace dmla {
 
 // ---- split-KV combine --------------------------------------------------------------------
-// One wave per (sequence, head), four per 256-thread block; lane l covers columns 4l + 256i.
 //   o = sum_s w_s o_s / sum_s w_s, w_s = exp(lse_s - max_s lse_s), lse = max + log(sum w)
-// over the first n_b splits; no finite lse leaves o = 0 and lse = -inf (max of the inputs);
-// a NaN lse makes o and lse NaN.  A split with lse = -inf is skipped whatever its o slot holds.
-// The weights are summed and applied in split order.  The common decode shape (at most 4
-// splits, d <= 512) issues every partial load before the first weight is known, so a wave
-// waits for one memory round trip instead of one per phase.
-constexpr int kCombineFast = 4;   // splits held in registers by the one-round-trip path
+// over the first n splits of a (sequence, head) pair; no finite lse leaves o = 0 and lse = -inf
+// (max of the inputs); a NaN lse makes o and lse NaN.  A split with lse = -inf is skipped whatever
+// its o slot holds.  kW waves share a pair: wave w adds the splits w, w + kW, .. in that order and
+// the kW sums meet in LDS, added in wave order, so the result does not depend on timing.
+// Bound: HBM latency.  A lane holds 16 bytes of a partial row, so one load instruction takes 1 KB
+// (a whole bf16 row), and kBatch rows are in flight per wave; the first batch goes out before the
+// lse values have arrived.  One wave per pair adding 79 splits one load at a time took 72 us at one
+// sequence of 5000 tokens and 128 heads (11.6 MB of partials); four waves and batches of 8 took
+// the decode call there from 93.4 to 28.1 us, and from 52.4 to 36.4 us at 16 sequences x 16 heads
+// (~17 splits each); at 64 sequences x 128 heads (3 splits) 115.4 -> 113.4 us.
+constexpr int kCombineFew = 4;     // splits of the usual large batch: one batch of 4 rows covers them
+constexpr int kCombineBatch = 8;   // rows in flight per wave otherwise
 
 template <typename T>
-__device__ __forceinline__ f32x4 load_part4(const T* p) {
-  if constexpr (std::is_same<T, float>::value) {
-    return *reinterpret_cast<const f32x4*>(p);
-  } else {
-    const bf16x4 x = *reinterpret_cast<const bf16x4*>(p);
-    return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
-  }
+struct PartVec {
+  static constexpr int kN = 16 / (int)sizeof(T);   // elements of one 16-byte load
+  T v[kN];
+};
+template <typename T>
+__device__ __forceinline__ PartVec<T> load_part(const T* p) {
+  return __builtin_bit_cast(PartVec<T>, *reinterpret_cast<const f32x4*>(p));
 }
 
-template <typename T>
+__device__ __forceinline__ float wave_max(float v) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  return v;
+}
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+template <typename T, int kW, int kBatch>
 __device__ __forceinline__ void combine_pair(const CombineArgs& a, const T* part, int b, int h, int n, int64_t s0,
-                                             int lane) {
+                                             int lane, int w, DMLA_LDS float* xch) {
+  constexpr int kN = PartVec<T>::kN;
+  constexpr int kCols = 64 * kN;   // columns of one pass
   const int64_t lbase = (a.split_base != nullptr ? s0 * a.lse_ss : (int64_t)b * a.lse_sb) + (int64_t)h * a.lse_sh;
-  const int64_t obase = (a.split_base != nullptr ? s0 * a.po_ss : (int64_t)b * a.po_sb) + (int64_t)h * a.po_sh;
+  const T* rows = part + (a.split_base != nullptr ? s0 * a.po_ss : (int64_t)b * a.po_sb) + (int64_t)h * a.po_sh;
   bf16* orow = a.o + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
-  // lse of split s < 64 sits in lane s; later splits are read again from memory
-  const float lv_lane = lane < n ? a.part_lse[lbase + (int64_t)lane * a.lse_ss] : kNegInf;
-  auto lse_of = [&](int s) -> float {
-    if (s < 64) return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv_lane), s));
-    return a.part_lse[lbase + (int64_t)s * a.lse_ss];
+  auto lse_chunk = [&](int c) { return c + lane < n ? a.part_lse[lbase + (int64_t)(c + lane) * a.lse_ss] : kNegInf; };
+  PartVec<T> x[kBatch];
+  // Rows w + kW u of the batch at s (wave-uniform); rows past n and columns past d read row 0 or
+  // column 0 instead and are not used.
+  auto load_batch = [&](int s, int cc) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) x[u] = load_part(rows + (int64_t)(s + kW * u < n ? s + kW * u : 0) * a.po_ss + cc);
   };
-  const bool fast = n >= 1 && n <= kCombineFast && a.d <= 512;
-  f32x4 pre[kCombineFast][2];
-  if (fast) {
-    // Unconditional loads (split 0 and column 0 stand in for the ones that do not exist), so
-    // that all of them are in flight together; the extra values are never used.
-#pragma unroll
-    for (int s = 0; s < kCombineFast; ++s)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int col = 4 * lane + 256 * i;
-        pre[s][i] = load_part4(part + obase + (int64_t)(s < n ? s : 0) * a.po_ss + (col < a.d ? col : 0));
-      }
-  }
-  float mx = kNegInf;
-  bool bad = false;   // a NaN lse (e.g. a split that met an invalid page) poisons the sequence
-  for (int s = 0; s < n; ++s) {
-    const float lv = lse_of(s);
-    bad = bad || lv != lv;
+  const float lv0 = lse_chunk(0);
+  if (n > 0) load_batch(w, kN * lane < a.d ? kN * lane : 0);
+  float mx = lv0;
+  bool nan_in = lv0 != lv0;   // a NaN lse (e.g. a split that met an invalid page) poisons the pair
+  for (int c = 64; c < n; c += 64) {
+    const float lv = lse_chunk(c);
+    nan_in = nan_in || lv != lv;
     mx = fmaxf(mx, lv);
   }
-  if (bad) {
+  if (__any(nan_in)) {
     const bf16 nb = (bf16)__builtin_nanf("");
-    for (int col = 4 * lane; col < a.d; col += 256) *reinterpret_cast<bf16x4*>(orow + col) = bf16x4{nb, nb, nb, nb};
-    if (lane == 0 && a.lse != nullptr) a.lse[(int64_t)b * a.H + h] = __builtin_nanf("");
+    for (int col = 4 * (lane + 64 * w); col < a.d; col += 256 * kW)
+      *reinterpret_cast<bf16x4*>(orow + col) = bf16x4{nb, nb, nb, nb};
+    if (lane == 0 && w == 0 && a.lse != nullptr) a.lse[(int64_t)b * a.H + h] = __builtin_nanf("");
     return;
   }
+  mx = wave_max(mx);
   const float mref = mx == kNegInf ? 0.f : mx;
-  float wsum = 0.f;
-  for (int s = 0; s < n; ++s) wsum += __expf(lse_of(s) - mref);
+  float wsum = __expf(lv0 - mref);
+  for (int c = 64; c < n; c += 64) wsum += __expf(lse_chunk(c) - mref);
+  wsum = wave_sum(wsum);
   const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-  auto store = [&](int col, f32x4 acc) {
-    acc *= inv;
-    bf16x4 w4;
-    w4[0] = (bf16)acc[0]; w4[1] = (bf16)acc[1]; w4[2] = (bf16)acc[2]; w4[3] = (bf16)acc[3];
-    *reinterpret_cast<bf16x4*>(orow + col) = w4;
-  };
-  if (fast) {
+  for (int col0 = 0; col0 < a.d; col0 += kCols) {
+    const int col = col0 + kN * lane, cc = col < a.d ? col : 0;
+    if (col0 > 0 && n > 0) load_batch(w, cc);
+    float acc[kN];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int col = 4 * lane + 256 * i;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < kN; ++e) acc[e] = 0.f;
+    for (int c = 0; c < n; c += 64) {
+      const float lv = c == 0 ? lv0 : lse_chunk(c);
+      const float wl = __expf(lv - mref) * inv;
+      const uint64_t live = __ballot(lv != kNegInf);
+      for (int s = c + w; s < min(n, c + 64); s += kW * kBatch) {
+        if (s != w) load_batch(s, cc);
 #pragma unroll
-      for (int s = 0; s < kCombineFast; ++s) {
-        const float lv = lse_of(s);
-        if (s < n && lv != kNegInf) acc += __expf(lv - mref) * pre[s][i];
+        for (int u = 0; u < kBatch; ++u) {
+          const int i = s - c + kW * u;
+          if (i >= 64 || !((live >> i) & 1)) continue;   // live holds no bit past n
+          const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wl), i));
+#pragma unroll
+          for (int e = 0; e < kN; ++e) acc[e] += ws * (float)x[u].v[e];
+        }
       }
-      if (col < a.d) store(col, acc);
     }
-  } else {
-    for (int col = 4 * lane; col < a.d; col += 256) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < n; ++s) {
-        const float lv = lse_of(s);
-        if (lv == kNegInf) continue;
-        acc += __expf(lv - mref) * load_part4(part + obase + (int64_t)s * a.po_ss + col);
+    if constexpr (kW == 1) {
+      if (col < a.d) {
+#pragma unroll
+        for (int q = 0; q < kN / 4; ++q) {
+          bf16x4 v;
+          v[0] = (bf16)acc[4 * q]; v[1] = (bf16)acc[4 * q + 1]; v[2] = (bf16)acc[4 * q + 2]; v[3] = (bf16)acc[4 * q + 3];
+          *reinterpret_cast<bf16x4*>(orow + col + 4 * q) = v;
+        }
       }
-      store(col, acc);
+    } else {
+#pragma unroll
+      for (int q = 0; q < kN / 4; ++q)
+        *reinterpret_cast<DMLA_LDS f32x4*>(xch + w * kCols + kN * lane + 4 * q) =
+            f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+      __syncthreads();
+      const int t = 64 * w + lane;
+      if (4 * t < kCols && col0 + 4 * t < a.d) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < kW; ++j) v += *reinterpret_cast<const DMLA_LDS f32x4*>(xch + j * kCols + 4 * t);
+        bf16x4 r;
+        r[0] = (bf16)v[0]; r[1] = (bf16)v[1]; r[2] = (bf16)v[2]; r[3] = (bf16)v[3];
+        *reinterpret_cast<bf16x4*>(orow + col0 + 4 * t) = r;
+      }
+      __syncthreads();   // the sums are read out before the next pass writes its own
     }
   }
-  if (lane == 0 && a.lse != nullptr) a.lse[(int64_t)b * a.H + h] = wsum > 0.f ? mref + __logf(wsum) : mx;
+  if (lane == 0 && w == 0 && a.lse != nullptr) a.lse[(int64_t)b * a.H + h] = wsum > 0.f ? mref + __logf(wsum) : mx;
 }
 
 // kPlan: the decode case, split_base and num_splits both given, so that both loads go out
-// together (one round trip before the partials' loads, not one per null check).
-template <bool kPlan>
+// together (one round trip before the partials' loads, not one per null check).  kW: waves per
+// pair, 1 (four pairs per 256-thread block) or 4.
+template <bool kPlan, int kW>
 __global__ void __launch_bounds__(256) lse_combine_kernel(CombineArgs a) {
+  __shared__ float xch[kW == 1 ? 1 : kW * 64 * 8];
   const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
   // 32-bit index math: the launcher checks B * H < 2^31
-  const unsigned pair = blockIdx.x * 4u + (unsigned)uniform(threadIdx.x >> 6);
+  const unsigned pair = kW == 1 ? blockIdx.x * 4u + (unsigned)wave : blockIdx.x;
   if (pair >= (unsigned)(a.B * a.H)) return;
   const int b = (int)(pair / (unsigned)a.H), h = (int)(pair - (unsigned)b * (unsigned)a.H);
   int n = a.max_splits;
@@ -123,27 +158,32 @@ __global__ void __launch_bounds__(256) lse_combine_kernel(CombineArgs a) {
     n = min(max(ns, 0), a.max_splits);
   } else {
     if (a.split_base != nullptr) s0 = a.split_base[b];
-    if (a.num_splits != nullptr) {
-      n = min(max(a.num_splits[b], 0), a.max_splits);
-    } else if (a.seqlens != nullptr) {
-      const int ctx = min(max(a.seqlens[b], 0), a.max_pages * a.page_size);
-      const int npages = (ctx + a.page_size - 1) / a.page_size;
-      n = max(1, (npages + a.pages_per_split - 1) / a.pages_per_split);
-    }
+    if (a.num_splits != nullptr) n = min(max(a.num_splits[b], 0), a.max_splits);
   }
   if (a.skip_single && n == 1) return;   // the decode kernel already wrote such rows itself
-  if (a.part_o16 != nullptr) combine_pair(a, a.part_o16, b, h, n, s0, lane);
-  else combine_pair(a, a.part_o, b, h, n, s0, lane);
+  DMLA_LDS float* x = (DMLA_LDS float*)xch;
+  const int w = kW == 1 ? 0 : wave;
+  auto run = [&](const auto* part) {
+    using T = std::remove_const_t<std::remove_pointer_t<decltype(part)>>;
+    if (kW == 1 && n <= kCombineFew) combine_pair<T, kW, kCombineFew>(a, part, b, h, n, s0, lane, w, x);
+    else combine_pair<T, kW, kCombineBatch>(a, part, b, h, n, s0, lane, w, x);
+  };
+  if (a.part_o16 != nullptr) run(a.part_o16);
+  else run(a.part_o);
 }
 
 int launch_lse_combine(const CombineArgs& a, hipStream_t stream, const char* what) {
   if (a.B == 0 || a.H == 0) return DMLA_OK;
-  if ((int64_t)a.B * a.H >= ((int64_t)1 << 31)) return fail(DMLA_ERR_UNSUPPORTED, "%s: B * H must be below 2^31", what);
-  const dim3 grid((unsigned)(((int64_t)a.B * a.H + 3) / 4));
-  if (a.split_base != nullptr && a.num_splits != nullptr)
-    hipLaunchKernelGGL(lse_combine_kernel<true>, grid, dim3(256), 0, stream, a);
-  else
-    hipLaunchKernelGGL(lse_combine_kernel<false>, grid, dim3(256), 0, stream, a);
+  const int64_t pairs = (int64_t)a.B * a.H;
+  if (pairs >= ((int64_t)1 << 31)) return fail(DMLA_ERR_UNSUPPORTED, "%s: B * H must be below 2^31", what);
+  // Four waves per pair where the pairs alone leave most of the chip's 8192 wave slots empty and a
+  // pair has more than a handful of splits.
+  const bool wide = pairs <= 2048 && a.mean_splits > kCombineFew;
+  const bool plan = a.split_base != nullptr && a.num_splits != nullptr;
+  const dim3 grid((unsigned)(wide ? pairs : (pairs + 3) / 4));
+  const auto kernel = wide ? (plan ? lse_combine_kernel<true, 4> : lse_combine_kernel<false, 4>)
+                           : (plan ? lse_combine_kernel<true, 1> : lse_combine_kernel<false, 1>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a);
   return check_launch(what);
 }
 
@@ -248,6 +288,7 @@ extern "C" int dmla_lse_combine(const float* part_o, const float* part_lse, cons
   a.o = static_cast<bf16*>(o);
   a.lse = lse;
   a.B = (int)B; a.H = (int)H; a.max_splits = (int)max_splits; a.d = (int)d;
+  a.mean_splits = (int)max_splits;
   a.po_sb = po_sb; a.po_ss = po_ss; a.po_sh = po_sh;
   a.lse_sb = lse_sb; a.lse_ss = lse_ss; a.lse_sh = lse_sh;
   a.o_sb = o_sb; a.o_sh = o_sh;

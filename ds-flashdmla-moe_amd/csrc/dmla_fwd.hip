@@ -1273,6 +1273,7 @@ int decode_launch(const void* q, const void* kv_pool, const int32_t* block_table
   c.o = p.o;
   c.lse = lse;
   c.B = (int)B; c.H = (int)H; c.max_splits = p.n_ranges + 1; c.d = kDv;
+  c.mean_splits = (int)((p.n_ranges + B - 1) / B);
   c.skip_single = 1;
   c.po_ss = H * kDv; c.po_sh = kDv;
   c.lse_ss = H; c.lse_sh = 1;

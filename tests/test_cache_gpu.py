@@ -108,3 +108,22 @@ def test_lse_combine_matches_oracle_and_full_attention(gpu):
     of, mf, lf = R.attention_exact(q[0].unsqueeze(1), keys[0:1], keys[0:1, :, :d], SCALE, False)
     assert_out_close(o[0], of[:, 0])
     assert (lse[0].cpu() - (mf + torch.log(lf))[:, 0]).abs().max().item() <= 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,S,d", [(1, 8, 5, 512), (2, 3, 31, 512), (1, 4, 32, 4), (3, 5, 33, 260), (1, 16, 64, 516),
+                                     (2, 2, 65, 512), (1, 3, 130, 256), (700, 3, 9, 64)])
+def test_lse_combine_many_splits(gpu, B, H, S, d):
+    """Split counts around the batches (8 rows, 4 waves, 64 lse values) on both sides of the rule
+    that gives a pair four waves (B * H <= 2048 and more than 4 splits); a split that holds
+    nothing (lse = -inf) is skipped even when its partial is NaN.  The result is a weighted mean in
+    fp32 rounded to bf16: within one bf16 rounding (2^-8) plus fp32 noise of the oracle."""
+    po = seeded((B, S, H, d), 11)
+    pl = seeded((B, S, H), 12, 2.0)
+    num = torch.tensor([1 + (7 * b) % S if b else S for b in range(B)], dtype=torch.int32)
+    pl[:, S // 2] = float("-inf")
+    ref_o, ref_lse = R.lse_combine(po, pl, num)
+    po[:, S // 2] = float("nan")
+    o, lse = ops.flash_dmla_lse_combine(po.to(gpu), pl.to(gpu), num.to(gpu), return_lse=True)
+    torch.testing.assert_close(o.float().cpu(), ref_o.float(), rtol=2.0 ** -7, atol=1e-5)
+    torch.testing.assert_close(lse.cpu(), ref_lse, rtol=1e-5, atol=1e-5)
