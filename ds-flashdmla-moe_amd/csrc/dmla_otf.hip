@@ -4,7 +4,8 @@
 //     O[b,h] = softmax(scale * Q[b,h] K_lat[b,h]^T (+ causal mask)) V_lat[b,h].
 // Shapes: Q [B,H,Sq,64], K and V [B,Sk,H,128], WK and WV [H,128,64], O [B,H,Sq,64].
 //
-// Workgroup = 8 waves on 512 query rows of one (batch, head); wave w owns rows 64w .. +63.
+// Workgroup = 8 waves on 512 query rows of one (batch, head); wave w owns rows 64w .. +63
+// (otf_fwd_short_kernel: fewer rows per workgroup, for short sequences).
 // Key tiles of 64 keys flow through a one-barrier-per-tile pipeline:
 //   * the raw K / V rows of tile t+2 are copied global -> LDS (direct copies, two stages);
 //   * tile t+1 is projected on MFMA: waves 0-3 compute K_lat^T (16 latent dims each, WK^T in
@@ -26,6 +27,7 @@
 // Softmax: in log2 units against a per-row reference max m_ref that only moves when a tile's
 // max exceeds it by more than kSlack (p <= 2^kSlack in between); moving it rescales O and l.  The exact running max is tracked beside it for the m / l outputs, which
 // follow the cache-latent forward's convention (natural-log units).
+#include <algorithm>
 #include <type_traits>
 
 #include "dmla_common.h"
@@ -41,17 +43,16 @@ constexpr int kOtfThreads = 64 * kOtfWaves;
 constexpr int kOtfRows = 64 * kOtfWaves;   // 512 query rows per workgroup
 constexpr int kOtfKeys = 64;               // keys per tile
 constexpr float kSlack = 8.0f;             // log2 slack of the reference max
-// LDS: W^T (2 x 64 x 128 bf16), raw K / V stages (2 x 2 x 64 x 128), K_lat hi and V_lat^T
-// (2 x 2 x 64 x 64), K_lat lo (2 x 64 x 64)
+// LDS: raw K / V stages (2 x 2 x 64 x 128 bf16), latent buffers (2 x [K_lat hi, V_lat^T, K_lat lo] of
+// 64 x 64).  WK and WV pass through the latent buffers once, before the first tile.
 constexpr int kWBytes = kDlat * kDin * 2;          // 16 KB
 constexpr int kRawBytes = kOtfKeys * kDin * 2;     // 16 KB
 constexpr int kLatBytes = kOtfKeys * kDlat * 2;    // 8 KB
-constexpr int kWOff = 0;                           // [WK^T, WV^T]
-constexpr int kRawOff = 2 * kWBytes;               // [stage][K, V]
-constexpr int kLatOff = kRawOff + 4 * kRawBytes;   // [buffer][K_lat, V_lat^T]
-constexpr int kLatLoOff = kLatOff + 4 * kLatBytes; // [buffer] K_lat lo
-constexpr int kOtfLds = kLatLoOff + 2 * kLatBytes; // 144 KB
-static_assert(kOtfLds <= 160 * 1024, "LDS budget");
+constexpr int kRawOff = 0;                         // [stage][K, V]
+constexpr int kLatOff = 4 * kRawBytes;             // [buffer][K_lat hi, V_lat^T, K_lat lo]
+constexpr int kBufBytes = 3 * kLatBytes;
+constexpr int kOtfLds = kLatOff + 2 * kBufBytes;   // 112 KB
+static_assert(2 * kWBytes <= 2 * kBufBytes, "W fits in the latent buffers");
 
 struct OtfParams {
   const bf16* q;
@@ -69,7 +70,8 @@ struct OtfParams {
   int64_t o_sb, o_sh, o_ss;
   int B, H, Sq, Sk, causal;
   float scale_log2;
-  int n_qt;                    // ceil(Sq / 512)
+  int n_qt;                    // row tiles per (batch, head)
+  int o_rows16;                // o strides are multiples of 8 elements (16-byte stores)
 };
 
 // Raw tile layout: [key (64)][16 chunks of 16 B], physical chunk = c ^ (key & 15): 16 lanes
@@ -78,6 +80,28 @@ __device__ __forceinline__ int raw_off(int key, int chunk) { return key * 256 + 
 // Latent tiles (K_lat [key][64 dims] and V_lat^T [dim][64 key positions]): 128-byte rows,
 // chunk c of row r at c ^ swz(r & 15) as in the cache-latent tiles.
 __device__ __forceinline__ int lat_off(int row, int chunk) { return row * 128 + 16 * (chunk ^ swz(row & 15)); }
+
+// WK[h] and WV[h] as they lie ([input (128)][64 latent dims], 128-byte rows) into the latent
+// buffers, one copy per 8 rows: chunk c of input row i at c ^ (i & 7).
+__device__ __forceinline__ void stage_w(const OtfParams& p, int h, unsigned lds_base, int wave, int lane) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int n = wave + 8 * j;
+    const int i = 8 * (n & 15) + (lane >> 3);
+    const bf16* w = (n < 16 ? p.wk : p.wv) + h * p.w_sh + i * p.w_si;
+    dma16_addr(w + 8 * ((lane & 7) ^ (i & 7)), lds_base + kLatOff + n * 1024);
+  }
+}
+// Eight inputs i0 .. i0 + 7 of latent dim d0 + (lane & 15), W^T as an MFMA operand, by two
+// transposed reads (i0, d0 per group of 16 lanes).  Written out transposed with 2-byte LDS writes
+// instead, W had cost each workgroup about 6 us before its first tile.
+__device__ __forceinline__ bf16x8 w_operand(const DMLA_LDS char* w, int i0, int d0, int lane) {
+  const int e = (lane & 15) >> 2, q = lane & 3;
+  auto at = [&](int i) {
+    return reinterpret_cast<const DMLA_LDS bf16x4*>(w + i * 128 + 16 * ((d0 / 8 + (q >> 1)) ^ (i & 7)) + 8 * (q & 1));
+  };
+  return concat(lds_read_tr16(at(i0 + e)), lds_read_tr16(at(i0 + 4 + e)));
+}
 
 __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[kOtfLds];
@@ -95,23 +119,7 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
   const int n_t = key_end > 0 ? (key_end + kOtfKeys - 1) / kOtfKeys : 0;
   const unsigned lds_base = lds_addr(lds);
 
-  // ---- WK^T and WV^T into LDS ([latent][input] rows of 256 B, same swizzle as raw tiles) ----
-  {
-    const bf16* wk = p.wk + h * p.w_sh;
-    const bf16* wv = p.wv + h * p.w_sh;
-    for (int idx = threadIdx.x; idx < kDin * kDlat / 8; idx += kOtfThreads) {
-      const int i = idx / (kDlat / 8), j8 = idx % (kDlat / 8);   // input dim i, latent dims 8 j8 ..
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(wk + i * p.w_si + 8 * j8);
-      const bf16x8 c = *reinterpret_cast<const bf16x8*>(wv + i * p.w_si + 8 * j8);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int j = 8 * j8 + e;
-        const int o = raw_off(j, i >> 3) + 2 * (i & 7);
-        *reinterpret_cast<DMLA_LDS bf16*>(lds + kWOff + o) = a[e];
-        *reinterpret_cast<DMLA_LDS bf16*>(lds + kWOff + kWBytes + o) = c[e];
-      }
-    }
-  }
+  stage_w(p, h, lds_base, wave, lane);
 
   // ---- raw K / V tile copies: 16 per tensor (4 keys x 256 B each), 4 per wave ----
   // Wave w copies tensor x = w / 4 (K, then V): copy c covers keys 4n .. 4n+3 with
@@ -157,7 +165,7 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
     }
   }
   wait_vmem();
-  __syncthreads();   // W^T written, raw tile 0 (and 1) landed
+  __syncthreads();   // W and raw tile 0 (and 1) landed
 
   // Projection operand of this wave: waves 0-3 hold WK^T rows 16 w .. +15 (A operand of
   // K_lat^T), waves 4-7 WV^T rows 16 (w-4) .. (B operand of V_lat); 4 k-steps of 32 input dims.
@@ -166,8 +174,11 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
   bf16x8 wreg[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks)
-    wreg[ks] = *reinterpret_cast<const DMLA_LDS bf16x8*>(lds + kWOff + (pk ? 0 : kWBytes) +
-                                                         raw_off(16 * pdb + l16, 4 * ks + g));
+    wreg[ks] = w_operand(lds + kLatOff + (pk ? 0 : kWBytes), 32 * ks + 8 * g, 16 * pdb, lane);
+  // Every wave holds its operands before the latent buffers take the first tile (lgkmcnt(0): the
+  // reads above are done).
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __syncthreads();
 
   // Project tile t (raw stage st) into latent buffer lb.  One wave-uniform branch for the
   // whole projection (a select per MFMA compiles to a branch around every MFMA).
@@ -175,7 +186,7 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
     auto proj = [&](auto is_k) {
       constexpr bool kK = decltype(is_k)::value;
       const DMLA_LDS char* raw = lds + kRawOff + (st * 2 + (kK ? 0 : 1)) * kRawBytes;
-      DMLA_LDS char* lat = lds + kLatOff + (lb * 2 + (kK ? 0 : 1)) * kLatBytes;
+      DMLA_LDS char* lat = lds + kLatOff + lb * kBufBytes + (kK ? 0 : kLatBytes);
       // The four key blocks' accumulations run interleaved (k-step outer), so consecutive MFMAs
       // are independent, and each k-step's raw reads go out one k-step ahead.  (Key block by key
       // block, every MFMA waited for the previous one's result and every read was awaited
@@ -217,7 +228,7 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
           const int key = 16 * kb + l16;
           const int o = lat_off(key, 2 * pdb + (g >> 1)) + 8 * (g & 1);
           *reinterpret_cast<DMLA_LDS bf16x4*>(lat + o) = hi;
-          *reinterpret_cast<DMLA_LDS bf16x4*>(lds + kLatLoOff + lb * kLatBytes + o) = lo;
+          *reinterpret_cast<DMLA_LDS bf16x4*>(lat + 2 * kLatBytes + o) = lo;
         } else {
           f16x4 v;
           v[0] = (_Float16)c[0]; v[1] = (_Float16)c[1]; v[2] = (_Float16)c[2]; v[3] = (_Float16)c[3];
@@ -255,9 +266,9 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
     // 32 KB of copies of all waves queue in the CU's vector-memory path ahead of the work.
     if (t + 2 < n_t) stage_raw(t + 2, t & 1);
 
-    const DMLA_LDS char* klat = lds + kLatOff + ((t & 1) * 2) * kLatBytes;
+    const DMLA_LDS char* klat = lds + kLatOff + (t & 1) * kBufBytes;
     const DMLA_LDS char* vlat = klat + kLatBytes;
-    const DMLA_LDS char* klo = lds + kLatLoOff + (t & 1) * kLatBytes;
+    const DMLA_LDS char* klo = klat + 2 * kLatBytes;
     // x[kb][rb] = S^T in log2 units minus the row's reference: keys 16 kb + 4g + i, row 16 rb +
     // l16.  The MFMA accumulators start at -m_ref (0 while a row has no reference), so x is the
     // exp2 argument as it leaves the matrix core.
@@ -386,10 +397,333 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_kernel(OtfParams p) {
   }
 }
 
+// ---- short sequences ------------------------------------------------------------------------
+// The kernel above needs 512-row tiles to spread the projection over; where these leave most CUs
+// without a workgroup (32 heads of 500 rows: 32 workgroups of 8 serial tiles), this one runs 256 or
+// 128 rows per workgroup on v_mfma_f32_32x32x16: a wave owns 32 query rows, and with kKS = 2 two
+// waves share them, each taking every tile's keys of one half and the pair's results merged at the
+// end.  Same tiles, stages, precision and softmax rules as above.  Bound: the latency of a tile's
+// chain (projection, scores, softmax, PV).  At 1 x 32 heads x 500 rows the kernel takes
+// 16.9 us with 128 rows per workgroup and 20.4 us with 256, against 35.8 us before (512 rows).
+//
+// LDS rows.  A 32x32 operand read (lane l: row l % 32, chunk 2 ks + l / 32 of 16 bytes) is served 16
+// lanes at a time, the lanes with equal bit 5 and equal parity of bits 2-4: 16 rows whose low four
+// bits all differ.
+//  * Raw K / V tiles: raw_off, chunk c of row r at c ^ (r & 15): the 16 rows of a group take 16
+//    different chunks, all 64 banks once.
+//  * Latent tiles (K_lat [key][64 dims], V_lat^T [dim][64 key positions]): rows of 8 chunks, two per
+//    256-byte bank line, chunk c of row r at c ^ ((r >> 1) & 7): the even (odd) rows of a group
+//    differ in bits 1-3.
+// The xor'd offsets of k-step ks are those of k-step 0 xor 32 ks.
+__device__ __forceinline__ int lat32_off(int row, int chunk) { return row * 128 + 16 * (chunk ^ ((row >> 1) & 7)); }
+
+template <int kKS>
+__global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_short_kernel(OtfParams p) {
+  constexpr int kRowWaves = kOtfWaves / kKS;
+  constexpr int kRows = 32 * kRowWaves;
+  constexpr int kKb = 2 / kKS;     // 32-key blocks of a tile per wave
+  __shared__ __attribute__((aligned(1024))) char smem[kOtfLds];
+  DMLA_LDS char* lds = (DMLA_LDS char*)smem;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int lane = lane_id();
+  const int l32 = lane & 31, hf = lane >> 5;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int kh = wave / kRowWaves;       // first key block of this wave (kKS = 2)
+  const int bh = (int)blockIdx.x % (p.B * p.H);
+  const int qt = p.n_qt - 1 - (int)blockIdx.x / (p.B * p.H);   // heaviest (latest) tiles first
+  const int b = bh / p.H, h = bh % p.H;
+  const int off = p.Sk - p.Sq;
+  const int row0 = qt * kRows + 32 * (wave % kRowWaves);       // this wave's first query row
+  const int last_row = min(p.Sq, qt * kRows + kRows) - 1;
+  const int key_end = p.causal ? min(p.Sk, last_row + off + 1) : p.Sk;
+  const int n_t = key_end > 0 ? (key_end + kOtfKeys - 1) / kOtfKeys : 0;
+  const unsigned lds_base = lds_addr(lds);
+
+  stage_w(p, h, lds_base, wave, lane);
+  // ---- raw K / V tile copies: as in the kernel above (wave w: tensor w / 4, keys 16 (w % 4) ..) ----
+  const int xw = wave >> 2;
+  const bf16* xbase = xw == 0 ? p.k + b * p.k_sb + h * p.k_sh : p.v + b * p.v_sb + h * p.v_sh;
+  const int64_t xss = xw == 0 ? p.k_ss : p.v_ss;
+  const unsigned raw_lane = (unsigned)((16 * (wave & 3) + g) * xss * 2);
+  auto stage_raw = [&](int t, int st) {
+    const unsigned ldst = lds_base + (st * 2 + xw) * kRawBytes + (wave & 3) * 4 * 1024;
+    if (t * kOtfKeys + kOtfKeys <= p.Sk) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        dma16(xbase + (int64_t)(t * kOtfKeys + 4 * c) * xss, raw_lane + 16u * (unsigned)(l16 ^ (4 * c + g)),
+              ldst + c * 1024);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int gk = min(t * kOtfKeys + 16 * (wave & 3) + 4 * c + g, p.Sk - 1);
+        dma16_addr(xbase + (int64_t)gk * xss + 8 * (l16 ^ (4 * c + g)), ldst + c * 1024);
+      }
+    }
+  };
+  if (n_t > 0) stage_raw(0, 0);
+  if (n_t > 1) stage_raw(1, 1);
+
+  // ---- Q rows of this wave as the B operand of S^T: qreg[ks] = Q[row0 + l32][16 ks + 8 hf ..]
+  bf16x8 qreg[4];
+  {
+    const bf16* qrow = p.q + b * p.q_sb + h * p.q_sh + (int64_t)min(row0 + l32, p.Sq - 1) * p.q_ss + 8 * hf;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qreg[ks] = *reinterpret_cast<const bf16x8*>(qrow + 16 * ks);
+  }
+  wait_vmem();
+  __syncthreads();   // W and raw tiles 0 and 1 landed
+  // This wave's W^T operand: wreg[ks] = W^T[32 dbp + l32][16 ks + 8 hf ..].
+  const int dbp = (wave >> 1) & 1, kbp = wave & 1;
+  bf16x8 wreg[8];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks)
+    wreg[ks] = w_operand(lds + kLatOff + (wave < 4 ? 0 : kWBytes), 16 * ks + 8 * hf, 32 * dbp + 16 * (g & 1), lane);
+  // Every wave holds its operands before the latent buffers take the first tile (lgkmcnt(0): the
+  // reads above are done).
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __syncthreads();
+
+  // One 32 x 32 block of the projection of a tile (raw stage st) into latent buffer lb: dims 32 dbp ..
+  // of keys 32 kbp .., K_lat (kK, waves 0-3) or V_lat (waves 4-7).
+  auto proj = [&](auto is_k, int st, int lb) {
+    constexpr bool kK = decltype(is_k)::value;
+    const int raw = (st * 2 + (kK ? 0 : 1)) * kRawBytes + raw_off(32 * kbp + l32, hf);
+    DMLA_LDS char* lat = lds + kLatOff + lb * kBufBytes + (kK ? 0 : kLatBytes);
+    f32x16 c = {};
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const bf16x8 xr = *reinterpret_cast<const DMLA_LDS bf16x8*>(lds + (raw ^ (32 * ks)));
+      if constexpr (kK) c = mfma32_bf16(wreg[ks], xr, c);   // K_lat^T[dim 32 dbp + 8a + 4 hf + i][key 32 kbp + l32]
+      else c = mfma32_bf16(xr, wreg[ks], c);                // V_lat[key 32 kbp + 8a + 4 hf + i][dim 32 dbp + l32]
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);   // all reads ahead of the MFMAs
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    const int lrow = lat32_off(kK ? 32 * kbp + l32 : 32 * dbp + l32, 0);   // chunk c of the row: xor 16 c
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      if constexpr (kK) {
+        // K_lat[key 32 kbp + l32][dims 32 dbp + 8a + 4 hf .. +3] times scale log2(e), as hi + lo
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float x = c[4 * a + i] * p.scale_log2;
+          hi[i] = (bf16)x;
+          lo[i] = (bf16)(x - (float)hi[i]);
+        }
+        const int o = (lrow ^ (64 * dbp + 16 * a)) + 8 * hf;
+        *reinterpret_cast<DMLA_LDS bf16x4*>(lat + o) = hi;
+        *reinterpret_cast<DMLA_LDS bf16x4*>(lat + 2 * kLatBytes + o) = lo;
+      } else {
+        f16x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (_Float16)c[4 * a + i];
+        // V_lat^T[dim][position]: key 32 kbp + 8a + 4 hf + i sits at position 32 kbp + 16 (a/2) +
+        // 8 hf + 4 (a%2) + i, the key order of the P operand (S^T C layout).
+        const int o = lrow ^ (64 * kbp + 16 * hf + 32 * (a >> 1));
+        *reinterpret_cast<DMLA_LDS f16x4*>(lat + o + 8 * (a & 1)) = v;
+      }
+    }
+  };
+  auto project = [&](int st, int lb) {
+    if (wave < 4) proj(std::true_type{}, st, lb);
+    else proj(std::false_type{}, st, lb);
+  };
+
+  f32x16 oacc[2] = {};   // O^T[dim 32 db + 8a + 4 hf + i][row0 + l32], element 4a + i
+  // Of the wave's keys, per own row l32: the reference max, the exact running max and the row sum
+  // (log2 units; the last two lane-partial).
+  float mref = kNegInf, mtrue = kNegInf, lsum = 0.f;
+  const int own_lim = p.causal ? min(row0 + l32 + off, p.Sk - 1) : p.Sk - 1;
+
+  if (n_t > 0) project(0, 0);
+  for (int t = 0; t < n_t; ++t) {
+    wait_vmem();
+    __syncthreads();   // latent tile t written, raw tile t+1 landed, raw stage t%2 and latent buffer (t+1)%2 free
+    if (t + 1 < n_t) project((t + 1) & 1, (t + 1) & 1);
+    if (t + 2 < n_t) stage_raw(t + 2, t & 1);
+
+    // Operand address of k-step ks in the tile's K_lat hi, V_lat^T (+ kLatBytes) and K_lat lo
+    // (+ 2 kLatBytes): the same row and chunk of each.
+    const int op0 = kLatOff + (t & 1) * kBufBytes + lat32_off(l32, hf);
+    const float nmr = mref == kNegInf ? 0.f : -mref;
+    f32x16 s[kKb];   // S^T minus the reference: key 32 (kh + kb) + 8a + 4 hf + i, row l32
+#pragma unroll
+    for (int kb = 0; kb < kKb; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[kb][i] = nmr;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < kKb; ++kb) {
+        const DMLA_LDS char* op = lds + (op0 ^ (32 * ks)) + (kh + kb) * 4096;
+        const bf16x8 lo = *reinterpret_cast<const DMLA_LDS bf16x8*>(op + 2 * kLatBytes);
+        const bf16x8 hi = *reinterpret_cast<const DMLA_LDS bf16x8*>(op);
+        s[kb] = mfma32_bf16(lo, qreg[ks], s[kb]);
+        s[kb] = mfma32_bf16(hi, qreg[ks], s[kb]);
+      }
+    // Six operand reads ahead of the MFMAs.
+    __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+    for (int i = 0; i < 8 * kKb - 6; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+    const int key0 = t * kOtfKeys;
+    if (key0 + kOtfKeys > p.Sk || (p.causal && key0 + kOtfKeys - 1 > row0 + off)) {
+#pragma unroll
+      for (int kb = 0; kb < kKb; ++kb) {
+        const int lim = own_lim - key0 - 32 * (kh + kb) - 4 * hf;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (8 * (i >> 2) + (i & 3) > lim) s[kb][i] = kNegInf;
+      }
+    }
+    float mx = kNegInf;
+#pragma unroll
+    for (int kb = 0; kb < kKb; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) mx = fmaxf(mx, fmaxf(s[kb][i], s[kb][i + 1]));
+    mx -= nmr;   // the max score in log2 units
+    mtrue = fmaxf(mtrue, mx);
+    if (__any(mx > mref + kSlack)) {
+      // Move the reference to the exact row max so far; rescale l and the O rows.
+      const float mnew = fmaxf(mref, half_max(mtrue));
+      const float f = mnew == kNegInf ? 1.f : fast_exp2(mref - mnew);   // 0 when mref = -inf
+      lsum *= f;
+      mref = mnew;
+      const float dn = (mnew == kNegInf ? 0.f : -mnew) - nmr;   // this tile's arguments move along
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+#pragma unroll
+        for (int kb = 0; kb < kKb; ++kb) s[kb][i] += dn;
+        oacc[0][i] *= f;
+        oacc[1][i] *= f;
+      }
+    }
+    const f16x2 ones = {(_Float16)1.f, (_Float16)1.f};
+#pragma unroll
+    for (int ks = 0; ks < 2 * kKb; ++ks) {
+      f16x8 pa;   // B operand of O^T += V_lat^T P^T: keys of the k-step in V_lat^T order
+#pragma unroll
+      for (int j = 0; j < 8; ++j) pa[j] = (_Float16)fast_exp2(s[ks >> 1][8 * (ks & 1) + j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) lsum = __builtin_amdgcn_fdot2(f16x2{pa[2 * j], pa[2 * j + 1]}, ones, lsum, false);
+      const int vop = (op0 ^ (32 * ks)) ^ (64 * kh);   // kh: 64 bytes (32 positions) along the row
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        const f16x8 vb = *reinterpret_cast<const DMLA_LDS f16x8*>(lds + vop + kLatBytes + db * 4096);
+        oacc[db] = mfma32_f16(vb, pa, oacc[db]);
+      }
+    }
+  }
+
+  // ---- merge of the two key halves: waves 4-7 hand theirs over through LDS ----
+  if constexpr (kKS == 2) {
+    __syncthreads();   // the last tile is read out
+    DMLA_LDS f32x4* ox = reinterpret_cast<DMLA_LDS f32x4*>(lds) + (wave % kRowWaves) * 9 * 64 + lane;
+    if (kh == 1) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        ox[64 * j] = f32x4{oacc[j >> 2][4 * (j & 3)], oacc[j >> 2][4 * (j & 3) + 1], oacc[j >> 2][4 * (j & 3) + 2],
+                           oacc[j >> 2][4 * (j & 3) + 3]};
+      ox[64 * 8] = f32x4{mref, mtrue, lsum, 0.f};
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    const f32x4 st = ox[64 * 8];
+    const float mnew = fmaxf(mref, st[0]);
+    const float f0 = mnew == kNegInf ? 1.f : fast_exp2(mref - mnew), f1 = mnew == kNegInf ? 0.f : fast_exp2(st[0] - mnew);
+    mref = mnew;
+    mtrue = fmaxf(mtrue, st[1]);
+    lsum = lsum * f0 + st[2] * f1;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const f32x4 o1 = ox[64 * j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        oacc[j >> 2][4 * (j & 3) + i] = oacc[j >> 2][4 * (j & 3) + i] * f0 + o1[i] * f1;
+    }
+  }
+
+  // ---- epilogue: row sums, statistics, normalised O ----
+  const float ltot = half_sum(lsum);
+  const float mrow = half_max(mtrue);
+  const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
+  const int r = row0 + l32;
+  if (r >= p.Sq) return;
+  if (hf == 0 && p.m) {
+    const int64_t idx = ((int64_t)b * p.H + h) * p.Sq + r;
+    const bool any = ltot > 0.f;
+    p.m[idx] = any ? mrow * kLn2 : kNegInf;
+    p.l[idx] = any ? ltot * fast_exp2(mref - mrow) : 0.f;
+  }
+  bf16* orow = p.o + b * p.o_sb + h * p.o_sh + (int64_t)r * p.o_ss;
+#pragma unroll
+  for (int db = 0; db < 2; ++db) {
+#pragma unroll
+    for (int ap = 0; ap < 2; ++ap) {
+      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+      typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+      bf16x4 x, y;   // dims 32 db + 16 ap + 4 hf .. +3 and 8 more
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = (bf16)(oacc[db][8 * ap + i] * inv);
+        y[i] = (bf16)(oacc[db][8 * ap + 4 + i] * inv);
+      }
+      if (p.o_rows16) {
+        // Swapping the halves' pieces leaves each lane 8 consecutive dims, 32 db + 16 ap + 8 hf ..
+        const u32x2 xu = __builtin_bit_cast(u32x2, x), yu = __builtin_bit_cast(u32x2, y);
+        u32x4 v;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const auto r2 = __builtin_amdgcn_permlane32_swap(xu[w], yu[w], false, false);
+          v[w] = r2[0];
+          v[2 + w] = r2[1];
+        }
+        *reinterpret_cast<u32x4*>(orow + 32 * db + 16 * ap + 8 * hf) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          orow[32 * db + 16 * ap + 4 * hf + i] = x[i];
+          orow[32 * db + 16 * ap + 8 + 4 * hf + i] = y[i];
+        }
+      }
+    }
+  }
+}
+
 }  // namespace
 }  // namespace dmla
 
 using namespace dmla;
+
+// Query rows per workgroup: 512 (otf_fwd_kernel) or 256 / 128 (otf_fwd_short_kernel).  A workgroup of
+// n key tiles takes about fixed_us + n tile_us, measured at 1 x 32 heads x 500 and 777 rows
+// (one workgroup per CU) and 2 x 32 x 4096 (all CUs busy): larger tiles cost less per row (the
+// projection is shared by more of them), smaller ones occupy more CUs and end sooner.  The estimate
+// is the larger of the chip's share of the work and the longest workgroup; the smallest wins.
+// Measured sides: 1 x 32 x 500 takes 34.4 / 20.4 / 16.9 us and 2 x 32 x 4096 234 / 291 / 401 us with
+// 512 / 256 / 128 rows.
+static int otf_tile(int64_t BH, int64_t Sq, int64_t Sk, int causal) {
+  static constexpr struct { int rows; double tile_us, fixed_us; } shapes[] = {
+      {kOtfRows, 2.9, 12.0}, {256, 2.0, 5.0}, {128, 1.5, 4.2}};
+  int best = 0;
+  double best_us = 0;
+  for (const auto& s : shapes) {
+    const double n_wg = (double)((Sq + s.rows - 1) / s.rows) * (double)BH;
+    // keys seen by a row tile: all of them, or on average those up to the middle tile's last row
+    const double rows = (double)std::min<int64_t>(Sq, s.rows);
+    const double keys = causal ? std::min((double)Sk, std::max(0.0, (double)(Sk - Sq) + 0.5 * ((double)Sq + rows))) : (double)Sk;
+    const double us = std::max(n_wg / device_cu_count() * (s.fixed_us + s.tile_us * keys / kOtfKeys),
+                               s.fixed_us + s.tile_us * (double)Sk / kOtfKeys);
+    if (best == 0 || us < best_us) { best = s.rows; best_us = us; }
+  }
+  return best;
+}
 
 extern "C" int dmla_fwd_onthefly(const void* q, const void* k, const void* v, const void* wk, const void* wv,
                                  void* o, float* m, float* l, int64_t B, int64_t H, int64_t Sq, int64_t Sk,
@@ -434,9 +768,12 @@ extern "C" int dmla_fwd_onthefly(const void* q, const void* k, const void* v, co
   p.B = (int)B; p.H = (int)H; p.Sq = (int)Sq; p.Sk = (int)Sk;
   p.causal = causal ? 1 : 0;
   p.scale_log2 = softmax_scale * kLog2e;
-  p.n_qt = (int)((Sq + kOtfRows - 1) / kOtfRows);
+  p.o_rows16 = mult8(o_sb) && mult8(o_sh) && mult8(o_ss);
+  const int rows = otf_tile(B * H, Sq, Sk, p.causal);
+  p.n_qt = (int)((Sq + rows - 1) / rows);
   const int64_t grid = (int64_t)p.n_qt * B * H;
   if (grid > 0x7fffffff) return fail(DMLA_ERR_UNSUPPORTED, "dmla_fwd_onthefly: grid too large");
-  hipLaunchKernelGGL(otf_fwd_kernel, dim3((unsigned)grid), dim3(kOtfThreads), 0, (hipStream_t)stream, p);
+  const auto kernel = rows == kOtfRows ? otf_fwd_kernel : rows == 256 ? otf_fwd_short_kernel<1> : otf_fwd_short_kernel<2>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kOtfThreads), 0, (hipStream_t)stream, p);
   return check_launch("dmla_fwd_onthefly");
 }

@@ -84,3 +84,41 @@ def test_otf_strided_views(gpu):
     o = ops.flash_dmla_fwd_onthefly(qb.to(gpu), kb.to(gpu), v.to(gpu), wk.to(gpu), wv.to(gpu), 0.125, True)
     o_ref, _, _ = R.dmla_fwd_onthefly(q, k, v, wk, wv, 0.125, True)
     assert_out_close(o, o_ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "B,H,Sq,Sk,causal",
+    [
+        # 128 rows per workgroup, two waves per row block: rows that see keys of one half only, a
+        # ragged last tile in either half, several row tiles
+        (1, 2, 20, 20, True),
+        (1, 2, 129, 95, False),
+        (1, 3, 257, 129, True),
+        (2, 32, 700, 700, True),
+        # 256 rows per workgroup
+        (16, 32, 130, 130, True),
+        (16, 32, 257, 600, False),
+        (3, 32, 513, 700, True),
+        # 512 rows per workgroup
+        (16, 32, 257, 257, True),
+        (16, 16, 300, 300, False),
+        (16, 32, 500, 1000, True),
+    ],
+)
+def test_otf_row_tiles(gpu, B, H, Sq, Sk, causal):
+    """The three workgroup shapes the launcher's estimate picks among, at their edges."""
+    _check(gpu, B, H, Sq, Sk, causal, seed=Sq + Sk, ref_device="gpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,S", [(1, 2, 70), (16, 32, 130), (16, 32, 257)])
+def test_otf_output_strides(gpu, B, H, S):
+    """Output strides that are no multiple of 8 elements (the C ABI takes any) store the same values."""
+    q, k, v, wk, wv = (t.to(gpu) for t in _inputs(B, H, S, S, seed=S))
+    ref = ops.flash_dmla_fwd_onthefly(q, k, v, wk, wv, 0.125, True)
+    o = torch.zeros((B, H, S, 67), dtype=torch.bfloat16, device=gpu)[..., :64]
+    P, s = ops._ptr, lambda t: tuple(t.stride())
+    ops._lib.call("dmla_fwd_onthefly", P(q), P(k), P(v), P(wk), P(wv), P(o), None, None, B, H, S, S, 128, 64, *s(q)[:3],
+                  *s(k)[:3], *s(v)[:3], *s(wk)[:2], *s(o)[:3], 0.125, 1, ops._stream(q))
+    assert torch.equal(o, ref)
