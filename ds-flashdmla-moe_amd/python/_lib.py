@@ -151,4 +151,6 @@ def check(name: str, rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(name, getattr(lib(), name)(*args))
+    rc = getattr(_lib or lib(), name)(*args)
+    if rc != DMLA_OK:
+        check(name, rc)

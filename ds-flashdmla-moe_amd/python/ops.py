@@ -29,12 +29,14 @@ D_V = 512
 PAGE_SIZE = 64
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# The calls below run in the time a small kernel takes (10-20 us), so the checks build no message and
+# no container unless they fail, and pointers and streams go to ctypes as plain integers.
+def _stream(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -43,6 +45,8 @@ def _require(cond: bool, msg: str) -> None:
 
 
 def _check_bf16(name: str, t: torch.Tensor, ndim: int) -> None:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.bfloat16 and t.dim() == ndim and t.stride(-1) == 1:
+        return
     _require(isinstance(t, torch.Tensor), f"{name} must be a tensor")
     _require(t.is_cuda, f"{name} must be a GPU tensor (the HIP kernels have no CPU path)")
     _require(t.dtype == torch.bfloat16, f"{name} must be bfloat16, got {t.dtype}")
@@ -52,9 +56,15 @@ def _check_bf16(name: str, t: torch.Tensor, ndim: int) -> None:
 
 def _same_device(**tensors: Optional[torch.Tensor]) -> None:
     """Raises unless every given tensor lives on one device (the kernels read them all there)."""
-    devs = {name: t.device for name, t in tensors.items() if t is not None}
-    _require(len(set(devs.values())) <= 1, "tensors must be on one device, got " +
-             ", ".join(f"{n} on {d}" for n, d in devs.items()))
+    first = None
+    for t in tensors.values():
+        if t is None:
+            continue
+        if first is None:
+            first = t.device
+        elif t.device != first:
+            raise ValueError("tensors must be on one device, got " +
+                             ", ".join(f"{n} on {t.device}" for n, t in tensors.items() if t is not None))
 
 
 def _check_fp16_range(name: str, t: torch.Tensor) -> None:
@@ -89,6 +99,8 @@ def _on_tensor_device(fn):
     def wrapped(*args, **kwargs):
         for a in (*args, *kwargs.values()):
             if isinstance(a, torch.Tensor) and a.is_cuda:
+                if a.get_device() == torch.cuda.current_device():
+                    break
                 with torch.cuda.device(a.device):
                     return fn(*args, **kwargs)
         return fn(*args, **kwargs)
@@ -115,8 +127,8 @@ def flash_dmla_fwd(
     _check_bf16("q", q, 4)
     _check_bf16("k_lat", k_lat, 3)
     B, H, Sq, Dqk = q.shape
-    _require(k_lat.shape[0] == B and k_lat.shape[2] == Dqk,
-             f"k_lat shape {tuple(k_lat.shape)} does not match q {tuple(q.shape)}")
+    if not (k_lat.shape[0] == B and k_lat.shape[2] == Dqk):
+        raise ValueError(f"k_lat shape {tuple(k_lat.shape)} does not match q {tuple(q.shape)}")
     _same_device(q=q, k_lat=k_lat)
     Sk = k_lat.shape[1]
     o = torch.empty((B, H, Sq, d_v), dtype=torch.bfloat16, device=q.device)
@@ -239,8 +251,10 @@ def flash_dmla_decode_paged(
     _require(cache_seqlens.is_contiguous(), "cache_seqlens must be contiguous")
     B, H, Dqk = q.shape
     num_pages, page, Dk = kv_pool.shape
-    _require(Dk == Dqk, f"kv_pool last dim {Dk} != q last dim {Dqk}")
-    _require(page == PAGE_SIZE, f"page size must be {PAGE_SIZE}, got {page}")
+    if Dk != Dqk:
+        raise ValueError(f"kv_pool last dim {Dk} != q last dim {Dqk}")
+    if page != PAGE_SIZE:
+        raise ValueError(f"page size must be {PAGE_SIZE}, got {page}")
     _require(block_table.shape[0] == B and cache_seqlens.shape[0] == B, "batch size mismatch")
     _same_device(q=q, kv_pool=kv_pool, block_table=block_table, cache_seqlens=cache_seqlens, plan=plan)
     max_pages = block_table.shape[1]
@@ -304,7 +318,8 @@ def flash_dmla_kv_append(
     _check_bf16("kv_pool", kv_pool, 3)
     _check_bf16("new_kv", new_kv, 3)
     for name, t, nd in (("block_table", block_table, 2), ("cache_seqlens", cache_seqlens, 1)):
-        _require(t.dtype == torch.int32 and t.dim() == nd and t.is_cuda, f"{name} must be a {nd}-D int32 GPU tensor")
+        if not (t.dtype == torch.int32 and t.dim() == nd and t.is_cuda):
+            raise ValueError(f"{name} must be a {nd}-D int32 GPU tensor")
     _require(block_table.stride(-1) == 1 and cache_seqlens.is_contiguous(), "index tensors must be contiguous")
     B, n_new, d = new_kv.shape
     num_pages, P, dk = kv_pool.shape
@@ -413,11 +428,13 @@ def flash_dmla_bwd(
     B, H, Sq, Dqk = q.shape
     Sk = k_lat.shape[1]
     _require(k_lat.shape[0] == B and k_lat.shape[2] == Dqk, "k_lat shape does not match q")
-    _require(tuple(o.shape) == (B, H, Sq, d_v), f"o must be [B, H, Sq, {d_v}]")
-    _require(tuple(do.shape) == (B, H, Sq, d_v), f"do must be [B, H, Sq, {d_v}]")
+    if not (tuple(o.shape) == (B, H, Sq, d_v)):
+        raise ValueError(f"o must be [B, H, Sq, {d_v}]")
+    if not (tuple(do.shape) == (B, H, Sq, d_v)):
+        raise ValueError(f"do must be [B, H, Sq, {d_v}]")
     for name, t in (("m", m), ("l", l)):
-        _require(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and tuple(t.shape) == (B, H, Sq),
-                 f"{name} must be a contiguous float32 GPU tensor [B, H, Sq]")
+        if not (t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and tuple(t.shape) == (B, H, Sq)):
+            raise ValueError(f"{name} must be a contiguous float32 GPU tensor [B, H, Sq]")
     _same_device(q=q, k_lat=k_lat, o=o, do=do, m=m, l=l)
     if check_range:
         for name, t in (("q", q), ("k_lat", k_lat), ("do", do)):
@@ -488,8 +505,8 @@ def flash_dmla_bwd_onthefly(
     _require(wk.stride() == wv.stride(), "wk and wv must share strides")
     _require(tuple(o.shape) == (B, H, Sq, Dl) and tuple(do.shape) == (B, H, Sq, Dl), "o and do must be [B, H, Sq, d_lat]")
     for name, t in (("m", m), ("l", l)):
-        _require(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and tuple(t.shape) == (B, H, Sq),
-                 f"{name} must be a contiguous float32 GPU tensor [B, H, Sq]")
+        if not (t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and tuple(t.shape) == (B, H, Sq)):
+            raise ValueError(f"{name} must be a contiguous float32 GPU tensor [B, H, Sq]")
     _same_device(q=q, k=k, v=v, wk=wk, wv=wv, o=o, do=do, m=m, l=l)
     scale = _scale(softmax_scale, Dl)
     if check_range:
