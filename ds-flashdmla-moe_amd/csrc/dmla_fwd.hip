@@ -27,6 +27,8 @@
 //  * Softmax in the exp2 domain against a per-row reference max fixed at the first tile: p
 //    stays below 2^kHeadroom, so O is never rescaled.  Scores climbing past that headroom
 //    trigger a recomputation of the row tile from a higher reference.
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -85,6 +87,8 @@ __device__ __forceinline__ void iteration_schedule() {
   __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 }
 
+constexpr int kMaxParts = 32;   // key ranges of a split prefill row tile
+
 struct MqaParams {
   const bf16* q;
   const bf16* kv;
@@ -113,6 +117,12 @@ struct MqaParams {
   int32_t* plan_out;   // with plan_inline: workgroup 0 stores the plan here (the combine reads it)
   bf16* part_o;        // [slots, H, 512] normalised partial outputs, rounded to bf16
   float* part_lse;     // [slots, H]
+  // prefill with split key ranges (PrefillSplit; slot = workgroup id)
+  float* part_o32;     // [slots, 64 rows, 512] normalised partial outputs
+  float2* part_ml;     // [slots, 64 rows] (max in log2 units, row sum relative to it)
+  int n_layers;
+  int first_rt[kMaxParts];        // first row tile with more than j parts
+  int layer_base[kMaxParts + 1];  // row tiles (of one batch element) in the layers before j
 };
 
 struct Work {
@@ -155,14 +165,15 @@ struct InlinePlan {
 constexpr int kDecodeLdsBytes = kLdsBytes + (int)sizeof(InlinePlan);
 static_assert(kDecodeLdsBytes <= 160 * 1024, "LDS budget (decode)");
 
-template <bool kDecode, int kHalf>
+template <bool kDecode, int kHalf, bool kSplit>
 __device__ __noinline__ void mqa_fwd_exact(const MqaParams* params, Work wk, DMLA_LDS char* lds, int wave, int lane);
 
 // kExact = false: the fast path, reference max = the row max of the first tile; on overflow it
 // hands the whole row tile to the kExact = true path, which first computes every row's exact
 // max in a scores-only pass and then runs the same pipeline against it.  The fast path never
 // contains the (register-hungry) retry code.
-template <bool kDecode, int kHalf, bool kExact>
+// kSplit: a prefill row tile whose keys are cut over several workgroups (mqa_fwd_split_kernel).
+template <bool kDecode, int kHalf, bool kExact, bool kSplit = false>
 __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams* params, const Work& wk,
                                              DMLA_LDS char* lds, const int wave, const int lane_arg) {
   // Per-lane values are derived here, per work item, rather than once per kernel: kept live
@@ -640,7 +651,7 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
       const i32x4 f0 = *reinterpret_cast<const DMLA_LDS i32x4*>(flags);
       const i32x4 f1 = *reinterpret_cast<const DMLA_LDS i32x4*>(flags + 4);
       if (((f0[0] | f0[1] | f0[2] | f0[3]) | (f1[0] | f1[1] | f1[2] | f1[3])) != 0) {
-        mqa_fwd_exact<kDecode, kHalf>(params, wk, lds, wave, lane);
+        mqa_fwd_exact<kDecode, kHalf, kSplit>(params, wk, lds, wave, lane);
         return;
       }
     }
@@ -665,7 +676,10 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
   }
   if (kh == 0 && g == 0 && own_row < nrows) {
     if constexpr (!kDecode) {
-      if (p.m != nullptr) {
+      if (kSplit && wk.nsplit > 1) {
+        p.part_ml[(int64_t)wk.slot * kRowsPerWG + 16 * rb + l16] =
+            make_float2(mt, mt == kNegInf ? 0.f : ltot * fast_exp2(mref - mt));
+      } else if (p.m != nullptr) {
         const int pos = fast_div(own_row, p.hdiv), head = own_row - pos * p.H;
         const int si = (b * p.H + head) * p.Sq + pos;
         p.m[si] = mt == kNegInf ? kNegInf : mt * kLn2;
@@ -681,6 +695,17 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
     }
   }
   const int col = 64 * wave + 4 * g;
+  if constexpr (kSplit) {
+    if (wk.nsplit > 1) {   // fp32 partials: the rows past the last one hold copies of the first
+      float* pp = p.part_o32 + ((int64_t)wk.slot * kRowsPerWG + l16) * kDv + col;
+#pragma unroll
+      for (int qg = 0; qg < 4; ++qg)
+#pragma unroll
+        for (int d = 0; d < kDbWave; ++d)
+          *reinterpret_cast<f32x4*>(pp + qg * 16 * kDv + 16 * d) = oacc[d][qg] * inv_l[qg];
+      return;
+    }
+  }
   if constexpr (!kDecode) {
     // O goes out as whole 1 KB rows: each wave writes its 64 x 64 block (scaled, bf16) into
     // the free ring slots as [row][512] with the 16-byte chunks of row r xor-swizzled by r % 16
@@ -749,7 +774,7 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
 // argument segment (MqaParams is the kernel's only argument), taken in the kernel itself: the
 // segment pointer is only defined inside kernels, and passing the parameters by reference
 // would copy them to scratch memory in every workgroup.
-template <bool kDecode, int kHalf>
+template <bool kDecode, int kHalf, bool kSplit>
 __device__ __noinline__ void mqa_fwd_exact(const MqaParams* params, Work wk, DMLA_LDS char* lds, int wave, int lane) {
   // Call arguments arrive in VGPRs; the staging code needs the wave-uniform values in SGPRs.
   const uint64_t pa = reinterpret_cast<uint64_t>(params);
@@ -762,7 +787,7 @@ __device__ __noinline__ void mqa_fwd_exact(const MqaParams* params, Work wk, DML
   wk.ctx = uniform(wk.ctx); wk.page_begin = uniform(wk.page_begin); wk.slot = uniform(wk.slot);
   lds = reinterpret_cast<DMLA_LDS char*>(static_cast<uintptr_t>(uniform((int)lds_addr(lds))));
   __syncthreads();
-  mqa_fwd_body<kDecode, kHalf, true>(p, &p, wk, lds, wave, lane);
+  mqa_fwd_body<kDecode, kHalf, true, kSplit>(p, &p, wk, lds, wave, lane);
 }
 
 // Exclusive prefix of one value per thread over the workgroup; `total` gets the sum.
@@ -939,6 +964,106 @@ __global__ __launch_bounds__(kThreads, 1) void mqa_fwd_kernel(MqaParams p) {
   }
 }
 
+// ---- prefill with split key ranges --------------------------------------------------------
+// A 64-row tile streams its keys serially, so a call with fewer row tiles than CUs (a chunk of 512
+// positions x 16 heads is 128) leaves CUs idle, and one with about as many ends with its longest
+// row tile.  There the host (prefill_split) cuts the key tiles of a row tile into parts of about the
+// same number of tiles, each a workgroup writing a normalised fp32 partial and its row statistics, merged
+// by prefill_combine_kernel; row tiles with one part write their rows themselves.
+// Workgroup id -> (b = id % B, layer j, row tile): layer j holds part j of the row tiles with more
+// than j parts, the last row tiles (those with the most keys) first.
+__device__ __forceinline__ int prefill_tiles(const MqaParams& p, int rt) {
+  const int last_row = min((rt + 1) * kRowsPerWG, p.H * p.Sq) - 1;
+  const int kend = p.causal ? min(p.Sk, fast_div(last_row, p.hdiv) + 1 + (p.Sk - p.Sq)) : p.Sk;
+  return (max(kend, 0) + kTileN - 1) / kTileN;
+}
+__device__ __forceinline__ int prefill_parts(const MqaParams& p, int rt) {
+  int n = 1;
+  for (int j = 1; j < p.n_layers; ++j) n += rt >= p.first_rt[j] ? 1 : 0;
+  return n;
+}
+
+__global__ __launch_bounds__(kThreads, 1) void mqa_fwd_split_kernel(MqaParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[kLdsBytes];
+  DMLA_LDS char* lds = (DMLA_LDS char*)smem;
+  const int lane = lane_id();
+  const int wave = uniform(threadIdx.x >> 6);
+  const int x = (int)blockIdx.x / p.B;
+  int j = 0;
+  while (j + 1 < p.n_layers && x >= p.layer_base[j + 1]) ++j;
+  const int rt = p.n_row_tiles - 1 - (x - p.layer_base[j]);
+  const int n = prefill_tiles(p, rt);
+  Work wk = {};
+  wk.b = (int)blockIdx.x % p.B;
+  wk.row0 = rt * kRowsPerWG;
+  wk.nsplit = prefill_parts(p, rt);
+  wk.tile_begin = (int)((int64_t)n * j / wk.nsplit);
+  wk.tile_end = (int)((int64_t)n * (j + 1) / wk.nsplit);
+  wk.slot = (int)blockIdx.x;
+  const MqaParams* params = (const MqaParams*)(__builtin_amdgcn_kernarg_segment_ptr());
+  if (((wave >> 1) & 1) == 0) mqa_fwd_body<false, 0, false, true>(p, params, wk, lds, wave, lane);
+  else mqa_fwd_body<false, 1, false, true>(p, params, wk, lds, wave, lane);
+}
+
+// o = sum_j w_j o_j / sum_j w_j with w_j = l_j 2^(m_j - M), M = max_j m_j; m = M, l = sum_j w_j.  One
+// wave per row of the row tiles with several parts, parts in order; lane l holds columns 8l .. 8l+7
+// and the rows of up to four parts are in flight together.
+__global__ __launch_bounds__(256) void prefill_combine_kernel(MqaParams p) {
+  const int lane = threadIdx.x & 63;
+  const int unit = (int)blockIdx.x >> 4;   // 16 workgroups of four rows per row tile
+  const int b = unit % p.B;
+  const int rt = p.n_row_tiles - 1 - unit / p.B;
+  const int rl = 4 * ((int)blockIdx.x & 15) + uniform(threadIdx.x >> 6);
+  const int r = rt * kRowsPerWG + rl;
+  if (r >= p.H * p.Sq) return;
+  const int n = prefill_parts(p, rt);
+  auto slot = [&](int j) { return (int64_t)(p.layer_base[j] + p.n_row_tiles - 1 - rt) * p.B + b; };
+  // the parts' (m, l) sit in lanes 0 .. n - 1
+  const int64_t own = slot(min(lane, n - 1));
+  float2 ml = p.part_ml[own * kRowsPerWG + rl];
+  if (lane >= n) ml = make_float2(kNegInf, 0.f);
+  float mx = ml.x;
+#pragma unroll
+  for (int o = 1; o < kMaxParts; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mx)));
+  const float w = mx == kNegInf ? 0.f : ml.y * fast_exp2(ml.x - mx);
+  float wsum = w;
+#pragma unroll
+  for (int o = 1; o < kMaxParts; o <<= 1) wsum += __shfl_xor(wsum, o, 64);
+  wsum = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wsum)));
+  f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+  for (int j0 = 0; j0 < n; j0 += 4) {
+    f32x4 x0[4], x1[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float* src = p.part_o32 + (slot(min(j0 + u, n - 1)) * kRowsPerWG + rl) * kDv + 8 * lane;
+      x0[u] = *reinterpret_cast<const f32x4*>(src);
+      x1[u] = *reinterpret_cast<const f32x4*>(src + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (j0 + u >= n) break;
+      const float wj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), j0 + u));
+      a0 += wj * x0[u];
+      a1 += wj * x1[u];
+    }
+  }
+  const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+  bf16x8 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = (bf16)(a0[i] * inv);
+    v[4 + i] = (bf16)(a1[i] * inv);
+  }
+  const int pos = fast_div(r, p.hdiv), head = r - pos * p.H;
+  *reinterpret_cast<bf16x8*>(p.o + b * p.o_sb + head * p.o_sh + pos * p.o_ss + 8 * lane) = v;
+  if (lane == 0 && p.m != nullptr) {
+    const int si = (b * p.H + head) * p.Sq + pos;
+    p.m[si] = mx == kNegInf ? kNegInf : mx * kLn2;
+    p.l[si] = wsum;
+  }
+}
+
 // One workgroup computes the decode plan (layout above) from the context lengths.  The arrays
 // the binary searches read are mirrored in LDS when they fit (the common case), so every
 // dependent step is an LDS access rather than a global memory round trip.
@@ -1097,12 +1222,92 @@ int64_t decode_ranges(int64_t B, int64_t H, int64_t max_pages) {
 
 using namespace dmla;
 
-extern "C" int dmla_fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, float* l,
-                                     int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk,
-                                     int64_t d_v, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                                     int64_t k_sb, int64_t k_ss, int64_t o_sb, int64_t o_sh,
-                                     int64_t o_ss, float softmax_scale, int causal,
-                                     dmla_stream_t stream) {
+namespace dmla {
+namespace {
+
+struct PrefillSplit {
+  int n_layers;                    // most parts of a row tile; 1: no split
+  int first_rt[kMaxParts];
+  int layer_base[kMaxParts + 1];
+  int64_t slots() const { return layer_base[n_layers]; }   // per batch element
+};
+
+int64_t prefill_tiles_host(int64_t H, int64_t Sq, int64_t Sk, int causal, int64_t rt) {
+  const int64_t last_pos = (std::min<int64_t>((rt + 1) * kRowsPerWG, H * Sq) - 1) / H;
+  const int64_t kend = causal ? std::min(Sk, last_pos + 1 + (Sk - Sq)) : Sk;
+  return (std::max<int64_t>(kend, 0) + kTileN - 1) / kTileN;
+}
+
+// Whether and how to split the key ranges of a prefill.  A workgroup of n key tiles takes about
+// kFixedUs + n kTileUs (measured: prologue and epilogue, and the tile loop), a merge kMergeUs,
+// kMergePartUs per part of a row and 4 KB of traffic per row and part at ~4 TB/s.  Unsplit, some CU
+// runs j + 1 workgroups at least as long as the (j CUs)-th longest.  Only calls with at most four
+// row tiles per CU are considered: past that the grid balances itself.  Measured sides (16 heads,
+// causal): 512 of 8192 positions 201 us unsplit, 135 in two parts, 156 in three; 4 of 8000 192 us
+// unsplit, 32 in 16 parts; 1024 of 1024 (row tiles of 1 to 32 tiles, one per CU) 32 us unsplit, 43
+// with the longest cut in two.
+constexpr double kFixedUs = 5.5, kTileUs = 0.85, kMergeUs = 4.0, kMergePartUs = 0.4;
+PrefillSplit prefill_split(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int causal) {
+  PrefillSplit sp = {};
+  const int64_t n_rt = (H * Sq + kRowsPerWG - 1) / kRowsPerWG, cus = device_cu_count();
+  sp.n_layers = 1;
+  sp.layer_base[1] = (int)n_rt;
+  if (n_rt * B > 4 * cus) return sp;
+  auto tiles = [&](int64_t rt) { return prefill_tiles_host(H, Sq, Sk, causal, rt); };
+  const int64_t nmax = tiles(n_rt - 1);
+  // at most 64 row tiles stand for all of them
+  const int64_t step = (n_rt + 63) / 64;
+  double total = 0;
+  int64_t samples = 0;
+  for (int64_t rt = n_rt - 1; rt >= 0; rt -= step, ++samples) total += (double)tiles(rt);
+  const double mean = total / (double)samples;
+  double best = 0;
+  for (int64_t j = 0; j * cus < n_rt * B; ++j)
+    best = std::max(best, (double)(j + 1) * (kFixedUs + kTileUs * (double)tiles(n_rt - 1 - j * cus / B)));
+  best = 0.92 * std::max(best, (double)(n_rt * B) * (kFixedUs + kTileUs * mean) / (double)cus);
+  int64_t best_t = 0;
+  static constexpr int kTry[] = {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
+  for (int s : kTry) {
+    const int64_t t = (nmax + s - 1) / s;
+    if (t < 4) break;
+    double parts = 0, merged = 0;
+    for (int64_t rt = n_rt - 1; rt >= 0; rt -= step) {
+      const int64_t np = std::max<int64_t>(1, (tiles(rt) + t - 1) / t);
+      parts += (double)np;
+      if (np > 1) merged += (double)np;
+    }
+    const double scale = (double)n_rt * (double)B / (double)samples;
+    const double wgs = parts * scale;
+    const double rounds = std::max(1.0, std::ceil(wgs / (double)cus - 0.01));
+    const double part_us = kFixedUs + kTileUs * mean * (double)samples / parts;
+    const double us = std::max(kFixedUs + kTileUs * (double)t, rounds * part_us) + kMergeUs + kMergePartUs * (double)s +
+                      merged * scale * kRowsPerWG * 4096.0 / 4e6;
+    if (us < best) { best = us; best_t = t; }
+  }
+  if (best_t == 0) return sp;
+  sp.n_layers = (int)std::min<int64_t>((nmax + best_t - 1) / best_t, kMaxParts);
+  int64_t base = 0;
+  for (int j = 0; j < sp.n_layers; ++j) {
+    int64_t lo = 0, hi = n_rt;   // first row tile with more than j parts: tiles > j best_t (all have part 0)
+    while (j > 0 && lo < hi) {
+      const int64_t mid = (lo + hi) / 2;
+      if (tiles(mid) > j * best_t) hi = mid; else lo = mid + 1;
+    }
+    sp.first_rt[j] = (int)lo;
+    sp.layer_base[j] = (int)base;
+    base += n_rt - lo;
+  }
+  sp.layer_base[sp.n_layers] = (int)base;
+  return sp;
+}
+
+int64_t prefill_slot_bytes() { return kRowsPerWG * (int64_t)(kDv * 4 + 8); }
+
+// Both prefill entry points; a workspace of the split's size (dmla_fwd_workspace_bytes) lets it run.
+int fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, float* l, int64_t B, int64_t H, int64_t Sq,
+                     int64_t Sk, int64_t d_qk, int64_t d_v, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
+                     int64_t k_ss, int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale, int causal,
+                     bool split, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   clear_error();
   if (!q || !k_lat || !o) return fail(DMLA_ERR_INVALID_ARG, "dmla_fwd_cache_latent: null q/k_lat/o");
   if ((m == nullptr) != (l == nullptr))
@@ -1142,10 +1347,61 @@ extern "C" int dmla_fwd_cache_latent(const void* q, const void* k_lat, void* o, 
   p.n_row_tiles = (int)((rows + kRowsPerWG - 1) / kRowsPerWG);
   const int64_t grid = (int64_t)p.n_row_tiles * B;
   if (grid > 0x7fffffff) return fail(DMLA_ERR_UNSUPPORTED, "dmla_fwd_cache_latent: grid too large");
-  hipLaunchKernelGGL(mqa_fwd_kernel<false>, dim3((unsigned)grid), dim3(kThreads), 0,
-                     (hipStream_t)stream, p);
-  return check_launch("dmla_fwd_cache_latent");
+  PrefillSplit sp = {};
+  if (split) sp = prefill_split(B, H, Sq, Sk, p.causal);
+  if (sp.n_layers <= 1) {
+    hipLaunchKernelGGL(mqa_fwd_kernel<false>, dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
+    return check_launch("dmla_fwd_cache_latent");
+  }
+  const int64_t slots = sp.slots() * B;
+  if (workspace == nullptr || workspace_bytes < slots * prefill_slot_bytes())
+    return fail(DMLA_ERR_WORKSPACE, "dmla_fwd_cache_latent_ws: workspace of %lld bytes needed (got %lld)",
+                (long long)(slots * prefill_slot_bytes()), (long long)workspace_bytes);
+  if (!aligned16(workspace)) return fail(DMLA_ERR_INVALID_ARG, "dmla_fwd_cache_latent_ws: workspace must be 16-byte aligned");
+  p.part_o32 = static_cast<float*>(workspace);
+  p.part_ml = reinterpret_cast<float2*>(p.part_o32 + slots * kRowsPerWG * kDv);
+  p.n_layers = sp.n_layers;
+  for (int j = 0; j < sp.n_layers; ++j) p.first_rt[j] = sp.first_rt[j];
+  for (int j = 0; j <= sp.n_layers; ++j) p.layer_base[j] = sp.layer_base[j];
+  hipLaunchKernelGGL(mqa_fwd_split_kernel, dim3((unsigned)slots), dim3(kThreads), 0, stream, p);
+  const int64_t merged = (p.n_row_tiles - sp.first_rt[1]) * B;
+  hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)(16 * merged)), dim3(256), 0, stream, p);
+  return check_launch("dmla_fwd_cache_latent_ws");
 }
+
+}  // namespace
+}  // namespace dmla
+
+extern "C" int dmla_fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, float* l,
+                                     int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk,
+                                     int64_t d_v, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                                     int64_t k_sb, int64_t k_ss, int64_t o_sb, int64_t o_sh,
+                                     int64_t o_ss, float softmax_scale, int causal,
+                                     dmla_stream_t stream) {
+  return fwd_cache_latent(q, k_lat, o, m, l, B, H, Sq, Sk, d_qk, d_v, q_sb, q_sh, q_ss, k_sb, k_ss, o_sb, o_sh, o_ss,
+                          softmax_scale, causal, false, nullptr, 0, (hipStream_t)stream);
+}
+
+extern "C" int64_t dmla_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk, int64_t d_v,
+                                            int causal) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || d_qk != kDqk || d_v != kDv) return 0;
+  if (B > ((int64_t)1 << 30) || H > ((int64_t)1 << 30) || Sq > ((int64_t)1 << 30) || H * Sq > ((int64_t)1 << 30) ||
+      Sk > ((int64_t)1 << 30))
+    return 0;
+  const PrefillSplit sp = prefill_split(B, H, Sq, Sk, causal ? 1 : 0);
+  return sp.n_layers > 1 ? sp.slots() * B * prefill_slot_bytes() : 0;
+}
+
+extern "C" int dmla_fwd_cache_latent_ws(const void* q, const void* k_lat, void* o, float* m, float* l,
+                                        int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk,
+                                        int64_t d_v, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                                        int64_t k_sb, int64_t k_ss, int64_t o_sb, int64_t o_sh,
+                                        int64_t o_ss, float softmax_scale, int causal, void* workspace,
+                                        int64_t workspace_bytes, dmla_stream_t stream) {
+  return fwd_cache_latent(q, k_lat, o, m, l, B, H, Sq, Sk, d_qk, d_v, q_sb, q_sh, q_ss, k_sb, k_ss, o_sb, o_sh, o_ss,
+                          softmax_scale, causal, true, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
 
 // Bytes of a decode plan for this batch on the current device (a multiple of 256).
 extern "C" int64_t dmla_decode_plan_bytes(int64_t B, int64_t H, int64_t max_pages_per_seq) {

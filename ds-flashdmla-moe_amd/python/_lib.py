@@ -53,6 +53,14 @@ SIGNATURES = {
         + [_i64] * 8  # q_sb q_sh q_ss k_sb k_ss o_sb o_sh o_ss
         + [_f32, _int, _ptr],  # scale, causal, stream
     ),
+    "dmla_fwd_workspace_bytes": (_i64, [_i64] * 6 + [_int]),  # B H Sq Sk d_qk d_v causal
+    "dmla_fwd_cache_latent_ws": (
+        _int,
+        [_ptr, _ptr, _ptr, _ptr, _ptr]  # q, k_lat, o, m, l
+        + [_i64] * 6  # B, H, Sq, Sk, d_qk, d_v
+        + [_i64] * 8  # q_sb q_sh q_ss k_sb k_ss o_sb o_sh o_ss
+        + [_f32, _int, _ptr, _i64, _ptr],  # scale, causal, workspace, workspace_bytes, stream
+    ),
     "dmla_fwd_onthefly": (
         _int,
         [_ptr] * 8  # q, k, v, wk, wv, o, m, l

@@ -68,6 +68,23 @@ int dmla_fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, f
                           float softmax_scale, int causal, dmla_stream_t stream);
 
 /*
+ * dmla_fwd_cache_latent with a workspace, for calls whose row tiles leave CUs idle (a chunk of a long
+ * prompt, a few short prompts): the keys of a row tile are cut over several workgroups, whose fp32
+ * partials and row statistics a second kernel merges.  Same arguments, results and checks;
+ * dmla_fwd_workspace_bytes gives the bytes needed on the current device (16-byte aligned device
+ * memory, contents ignored), 0 where the call would not be split and runs as
+ * dmla_fwd_cache_latent does (the workspace may then be NULL).
+ */
+int64_t dmla_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk,
+                                 int64_t d_v, int causal);
+int dmla_fwd_cache_latent_ws(const void* q, const void* k_lat, void* o, float* m, float* l,
+                             int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk,
+                             int64_t d_v, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
+                             int64_t k_ss, int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                             float softmax_scale, int causal, void* workspace,
+                             int64_t workspace_bytes, dmla_stream_t stream);
+
+/*
  * On-the-fly DMLA forward (prefill): per-head latent projections inside the kernel.
  * Replaces: fa2_forward (csrc/attention/fa2_fwd.cu:139-156) in the on-the-fly mode of
  * README.md:14 -- the role of the absent csrc/attention/fa2_dmla_fwd.cu (README.md:45).

@@ -105,3 +105,34 @@ def test_fwd_is_deterministic(gpu):
     b = ops.flash_dmla_fwd(q.to(gpu), k.to(gpu), 512, SCALE, True)
     for x, y in zip(a, b):
         assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "B,H,Sq,Sk,causal,split",
+    [
+        (1, 16, 4, 4100, True, True),      # one row tile, many parts, ragged last tile
+        (1, 16, 512, 2000, True, True),    # a chunk: every row tile in equal parts
+        (1, 1, 700, 700, True, True),      # one to several parts; parts in which rows see no key
+        (1, 128, 33, 3000, False, True),   # non-causal, ragged row tile
+        (2, 3, 100, 1500, True, True),
+        (1, 1, 1300, 900, True, True),     # leading rows without keys
+        (1, 16, 333, 333, True, False),    # just as well on as many CUs as it has row tiles
+    ],
+)
+def test_fwd_split_key_ranges(gpu, B, H, Sq, Sk, causal, split):
+    """Calls that leave CUs idle cut their key ranges over several workgroups (the workspace
+    query says which); the merge keeps fp32 partials, so the bars are the unsplit ones."""
+    q = seeded((B, H, Sq, 576), 70 + Sq, 0.5, torch.bfloat16).to(gpu)
+    k = seeded((B, Sk, 576), 71 + Sk, 0.5, torch.bfloat16).to(gpu)
+    assert (ops._lib.lib().dmla_fwd_workspace_bytes(B, H, Sq, Sk, 576, 512, int(causal)) > 0) == split
+    o, m, l = ops.flash_dmla_fwd(q, k, 512, SCALE, causal)
+    o_ref, m_ref, l_ref = R.dmla_fwd_cache_latent(q.float(), k.float(), 512, SCALE, causal)
+    assert_out_close(o, o_ref)
+    assert_stats_close(m, l, m_ref, l_ref)
+    # scores growing along the keys pass the reference max's headroom: the exact path, per part
+    k2 = (k.float() * torch.linspace(0.1, 30.0, Sk, device=gpu).view(1, Sk, 1)).to(torch.bfloat16)
+    o, m, l = ops.flash_dmla_fwd(q, k2, 512, SCALE, causal)
+    o_ref, m_ref, l_ref = R.dmla_fwd_cache_latent(q.float(), k2.float(), 512, SCALE, causal)
+    assert_stats_close(m, l, m_ref, l_ref)
+    assert ((o.float() - o_ref).abs().max() / o_ref.abs().max()).item() <= 1e-2
