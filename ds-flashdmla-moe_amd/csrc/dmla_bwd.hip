@@ -145,8 +145,10 @@ __host__ __device__ inline PairPlan pair_plan(int causal, int Sq, int Sk, int H,
   pp.total = pp.steps_a + (pp.kb_b != pp.kb_a ? max(0, rt_end - pp.first_b) : 0);
   return pp;
 }
+// First step of segment j (j = parts: the end).  total <= 2^26 steps and j < parts <= kMaxParts = 64
+// keep the product below 2^32.
 __host__ __device__ inline int part_begin(int total, int parts, int j) {
-  return (int)(((int64_t)total * j) / parts);
+  return j == parts ? total : (int)((unsigned)total * (unsigned)j / (unsigned)parts);
 }
 
 // Slot of C-order lane c in a stored 16x16 dS' block (8 bytes per slot): bit 2 of the lane
@@ -621,7 +623,9 @@ bwd_dkdv_kernel(BwdParams p) {
 // C-order blocks through ds_read_b64_tr_b16, K^T (B operand) with b128 reads.  Tiles flow
 // through a 3-slot ring: the copies of tile kt+2 go out between the MFMAs of tile kt, so the
 // dS' blocks (read from HBM) have two tiles of time to land.
-__device__ __forceinline__ void dk_reduce_unit(const BwdParams& p, int b, int kb, int kbl, int t);
+constexpr int kReduceThirds = 3;                    // the dK_lat reduction's units per 16 keys
+constexpr int kReduceUnits = 4 * kReduceThirds;     // and per 64-key block
+__device__ __forceinline__ void dk_reduce_unit(const BwdParams& p, int b, int kb, int kbl, int third, int t);
 
 __global__ void __launch_bounds__(kDqThreads, 1) bwd_dq_kernel(BwdParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[kDqLds];
@@ -632,10 +636,12 @@ __global__ void __launch_bounds__(kDqThreads, 1) bwd_dq_kernel(BwdParams p) {
   const int g_end = (p.rt_end + 3) / 4;
   const int n_dq = p.B * (g_end - p.rt_begin / 4);
   if ((int)blockIdx.x >= n_dq) {
-    // Past the dQ tiles: the dK_lat reduction, two (b, key block, column quarter) units per
+    // Past the dQ tiles: the dK_lat reduction, two (b, key block, 16 keys, column third) units per
     // workgroup, one per 256 threads.  These workgroups start as the dQ tiles drain.
     const int u = 2 * ((int)blockIdx.x - n_dq) + (int)(threadIdx.x >> 8);
-    if (u < 4 * p.n_kb * p.B) dk_reduce_unit(p, u / (4 * p.n_kb), (u / 4) % p.n_kb, u % 4, (int)(threadIdx.x & 255));
+    const int kbu = u / kReduceUnits, part = u % kReduceUnits;
+    if (kbu < p.n_kb * p.B)
+      dk_reduce_unit(p, kbu / p.n_kb, kbu % p.n_kb, part / kReduceThirds, part % kReduceThirds, (int)(threadIdx.x & 255));
     return;
   }
   const int b = (int)blockIdx.x % p.B;
@@ -791,42 +797,54 @@ __global__ void __launch_bounds__(kDqThreads, 1) bwd_dq_kernel(BwdParams p) {
 }
 
 // ---- 5. dK_lat = sum of the segment partials ------------------------------------------------
-// One unit per (batch, 64-key block, 16-key block), run by 256 threads of a workgroup past the
-// dQ tiles of bwd_dq_kernel (they start as those tiles drain; a launch of its own measured
-// 20 us, the shared launch ~5 us less in the traced sum).  The segments of the block are added
-// in part order, so the result does not depend on scheduling.  Thread t owns the 9 (column block,
-// lane) slots t + 256 r of the 16 keys and loads all 9 of a part together (a wave reads 1 KB per
-// slot), so each wave keeps 9 KB in flight instead of one dependent load per slot (33 -> 19 us
-// at config 5; two parts at a time measured no faster).
-constexpr int kReduceSlots = kCb * 64 / 256;
-static_assert(kReduceSlots * 256 == kCb * 64, "the reduction's slots cover the partial evenly");
+// One unit per (batch, 64-key block, 16-key block, third of the columns), run by 256 threads of a
+// workgroup past the dQ tiles of bwd_dq_kernel (they start as those tiles drain; a launch of its own
+// measured 20 us, the shared launch ~5 us less in the traced sum).  The segments of the block are
+// added in part order, so the result does not depend on scheduling.  Thread t owns the (column block,
+// lane) slots t + 256 r of the 16 keys in its third and loads kReduceBatch parts of them together:
+// what bounds a unit is memory latency, one round trip per batch.  With 9 slots (all columns) and one
+// part per round trip the dQ launch of 2 x 16 heads x 391 rows (32 parts) took 36.6 us, now 19.2.
+constexpr int kReduceSlots = kCb * 64 / 256 / kReduceThirds;
+constexpr int kReduceBatch = 4;
+static_assert(kReduceSlots * kReduceThirds * 256 == kCb * 64, "the reduction's slots cover the partial evenly");
 
-__device__ __forceinline__ void dk_reduce_unit(const BwdParams& p, int b, int kb, int kbl, int t) {
+__device__ __forceinline__ void dk_reduce_unit(const BwdParams& p, int b, int kb, int kbl, int third, int t) {
   const int pi = min(kb, p.n_kb - 1 - kb);
   const int ph = kb == pi ? 0 : 1;
   const PairPlan pp = pair_plan(p.causal, p.Sq, p.Sk, p.H, p.rt_begin, p.rt_end, p.n_kb, pi);
   const int iv_lo = ph == 0 ? 0 : pp.steps_a;
   const int iv_hi = ph == 0 ? pp.steps_a : pp.total;
   const int ln = t & 63;
+  // Parts that stored a partial for this phase: of the run j0 .. j1 - 1 that meets [iv_lo, iv_hi), those
+  // whose segment is not empty (a pair may have fewer steps than parts).
+  int j0 = 0, j1 = 0;
+  if (iv_lo < iv_hi) {
+    while (part_begin(pp.total, p.parts, j0 + 1) <= iv_lo) ++j0;
+    j1 = j0 + 1;
+    while (j1 < p.parts && part_begin(pp.total, p.parts, j1) < iv_hi) ++j1;
+  }
+  const f32x4* src = reinterpret_cast<const f32x4*>(p.part + ((int64_t)(b * p.parts * p.n_pairs + pi) * 2 + ph) * kPartFloats) +
+                     kbl * kCb * 64 + third * kReduceSlots * 256 + t;
+  const int64_t part_step = (int64_t)p.n_pairs * 2 * (kPartFloats / 4);
   f32x4 s[kReduceSlots];
 #pragma unroll
   for (int r = 0; r < kReduceSlots; ++r) s[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < p.parts; ++j) {
-    const int lo = part_begin(pp.total, p.parts, j), hi = part_begin(pp.total, p.parts, j + 1);
-    if (max(lo, iv_lo) >= min(hi, iv_hi)) continue;   // no partial stored for this phase
-    const int u = (b * p.parts + j) * p.n_pairs + pi;
-    const f32x4* src = reinterpret_cast<const f32x4*>(p.part + ((int64_t)u * 2 + ph) * kPartFloats) +
-                       kbl * kCb * 64 + t;
-    f32x4 v[kReduceSlots];
+  for (int j = j0; j < j1; j += kReduceBatch) {
+    f32x4 v[kReduceBatch][kReduceSlots];
 #pragma unroll
-    for (int r = 0; r < kReduceSlots; ++r) v[r] = src[256 * r];
+    for (int q = 0; q < kReduceBatch; ++q)
 #pragma unroll
-    for (int r = 0; r < kReduceSlots; ++r) s[r] += v[r];
+      for (int r = 0; r < kReduceSlots; ++r) v[q][r] = src[min(j + q, j1 - 1) * part_step + 256 * r];
+#pragma unroll
+    for (int q = 0; q < kReduceBatch; ++q)
+      if (j + q < j1 && part_begin(pp.total, p.parts, j + q) < part_begin(pp.total, p.parts, j + q + 1))
+#pragma unroll
+        for (int r = 0; r < kReduceSlots; ++r) s[r] += v[q][r];
   }
   const float unscale = exp2i(-grad_exponent(p.gmax));   // the partials carry 2^e
 #pragma unroll
   for (int r = 0; r < kReduceSlots; ++r) {
-    const int cb = (t >> 6) + 4 * r;
+    const int cb = (t >> 6) + 4 * (third * kReduceSlots + r);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int key = kb * kKeys + 16 * kbl + 4 * (ln >> 4) + i;
@@ -1017,7 +1035,7 @@ extern "C" int dmla_bwd_cache_latent(const void* q, const void* k_lat, const voi
   p.dk_acc = dk_fp32 ? static_cast<float*>(dk_lat) : reinterpret_cast<float*>(ws + pl.off_acc);
   // The dQ launch holds a chunk's row groups plus the reduction's units, two per workgroup; a
   // dispatch counts its work-items in 32 bits.
-  if ((B * (int64_t)pl.n_groups + 2 * (int64_t)pl.n_kb * B) * kDqThreads > 0xffffffffll)
+  if ((B * (int64_t)pl.n_groups + kReduceUnits / 2 * (int64_t)pl.n_kb * B) * kDqThreads > 0xffffffffll)
     return fail(DMLA_ERR_UNSUPPORTED, "dmla_bwd_cache_latent: grid too large");
 
   hipStream_t s = (hipStream_t)stream;
@@ -1038,7 +1056,7 @@ extern "C" int dmla_bwd_cache_latent(const void* q, const void* k_lat, const voi
     const int64_t grid_kv = 8 * ((c.n_items + 7) / 8);
     hipLaunchKernelGGL(bwd_dkdv_kernel, dim3((unsigned)grid_kv), dim3(kBwdThreads), 0, s, p);
     // dQ tiles, then the dK_lat reduction's units two per workgroup (bwd_dq_kernel)
-    const int64_t n_red = (int64_t)2 * pl.n_kb * B;
+    const int64_t n_red = (int64_t)(kReduceUnits / 2) * pl.n_kb * B;
     hipLaunchKernelGGL(bwd_dq_kernel, dim3((unsigned)(B * (c.g1 - c.g0) + n_red)), dim3(kDqThreads), 0, s, p);
     g0 = c.g1;
   }

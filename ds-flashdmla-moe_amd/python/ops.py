@@ -394,9 +394,10 @@ class FlashDMLACacheLatent(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         q, k_lat, o, m, l = ctx.saved_tensors
+        # dk_lat in its own dtype: the kernel rounds the fp32 sum last, as a cast of it would
         dq, dk_lat = flash_dmla_bwd(q, k_lat, o, do.to(torch.bfloat16).contiguous(), m, l, ctx.d_v,
-                                    ctx.softmax_scale, ctx.causal)
-        return dq, dk_lat.to(k_lat.dtype), None, None, None
+                                    ctx.softmax_scale, ctx.causal, dk_dtype=k_lat.dtype)
+        return dq, dk_lat, None, None, None
 
 
 @_on_tensor_device
