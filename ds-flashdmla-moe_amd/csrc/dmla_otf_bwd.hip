@@ -15,7 +15,7 @@
 //   otf_bwd_dkdv_kernel    per 128 keys: projects their K_lat and V_lat (also stored in fp16
 //                          for the dQ kernel), then dK_lat, dV_lat over the rows that see them;
 //   otf_bwd_dq_kernel      per 128 rows: dQ over the keys they see (S and dP recomputed);
-//   otf_bwd_wgrad_kernel   per (tensor, head, 1024 keys): dK / dV and a dWK / dWV partial;
+//   otf_bwd_wgrad_kernel   per (tensor, head, up to 1024 keys): dK / dV and a dWK / dWV partial;
 //   otf_bwd_wreduce_kernel sums the partials of each head in a fixed order.
 //
 // Precision.  dK_lat and dV_lat sum one term per row that sees a key, and through them dk, dv
@@ -49,7 +49,7 @@ constexpr int kIn = 128;                // raw K / V dims per head
 constexpr int kLat = 64;                // latent dims (Q, K_lat, V_lat, O)
 constexpr int kRowBlk = 128;            // dQ workgroup rows; row statistics are padded to a multiple
 constexpr int kKeyBlk = 128;            // dK/dV workgroup keys; keys are padded to a multiple
-constexpr int kChunk = 1024;            // keys per weight-gradient workgroup
+constexpr int kMaxChunk = 1024, kMinChunk = 128;   // keys per weight-gradient workgroup (OtfBwdPlan::chunk)
 constexpr int kTile = 32 * kLat * 2;    // one 32-row tile of 64 16-bit columns (4 KB)
 constexpr int kStage = 4 * kTile;       // 64 rows of two tensors (16 KB)
 constexpr int kRowStage = kStage + 512; // dK/dV stage: 64 rows of Q and dO, then their lse2 and -D
@@ -77,7 +77,7 @@ struct OtfBwdParams {
   int64_t dq_sb, dq_sh, dq_ss, dk_sb, dk_ss, dk_sh, dw_sh, dw_si;
   int B, H, Sq, Sk, causal;
   int Sqp, Skp;          // rows / keys padded to multiples of 128
-  int n_sc;              // 1024-key chunks per batch element (weight gradients)
+  int chunk, n_sc;       // keys per weight-gradient workgroup, chunks per batch element
   float scale, scale_log2;
   float* lse2;           // [B*H][Sqp]: (m + ln l) log2(e); padding and empty rows +inf
   float* nd;             // [B*H][Sqp]: -D = -rowsum(dO * O); padding rows 0
@@ -669,7 +669,7 @@ __global__ void __launch_bounds__(256, 3) otf_bwd_dq_kernel(OtfBwdParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Weight side: block = (tensor x in {K, V}, head h, batch b, chunk c of 1024 keys), grid
+// Weight side: block = (tensor x in {K, V}, head h, batch b, chunk c of p.chunk keys), grid
 // (n_sc, H, 2 B).  Per 64-key block (raw X rows and the dX_lat hi / lo planes copied global ->
 // LDS directly, one block ahead):
 //   dX^T[in][key] = W[in][:] dX_lat^T       wave w: keys 16 w .. +15 (A = W rows in registers,
@@ -690,7 +690,7 @@ __global__ void __launch_bounds__(256, 2) otf_bwd_wgrad_kernel(OtfBwdParams p) {
   const bf16* dxh = p.dxlat + 2 * x * plane + (size_t)bh * p.Skp * kLat;
   const bf16* dxl = dxh + plane;
   const int64_t dx_at = b * p.dk_sb + h * p.dk_sh;
-  const int key_lo = c * kChunk, key_hi = min(p.Sk, key_lo + kChunk);
+  const int key_lo = c * p.chunk, key_hi = min(p.Sk, key_lo + p.chunk);
   const int n_blk = (key_hi - key_lo + 63) / 64;
   const unsigned lbase = lds_addr(lds);
 
@@ -747,22 +747,45 @@ __global__ void __launch_bounds__(256, 2) otf_bwd_wgrad_kernel(OtfBwdParams p) {
       const bf16x8 lo0 = lds_bf16x8(dls + tt + row_operand_off(lane, rb, 0));
       const bf16x8 lo1 = lds_bf16x8(dls + tt + row_operand_off(lane, rb, 1));
       const int key = key_lo + 64 * blk + 16 * wave + l16;
+      const int64_t at = dx_at + (int64_t)key * p.dk_ss;
 #pragma unroll
-      for (int ib = 0; ib < 8; ++ib) {
-        f32x4 cacc = mfma_bf16(wa[ib][0], lo0, f32x4{0.f, 0.f, 0.f, 0.f});
-        cacc = mfma_bf16(wa[ib][0], h0, cacc);
-        cacc = mfma_bf16(wa[ib][1], lo1, cacc);
-        cacc = mfma_bf16(wa[ib][1], h1, cacc);    // dX^T[in 16 ib + 4 g + i][key]
-        if (key < key_hi) {
-          const int64_t at = dx_at + (int64_t)key * p.dk_ss + 16 * ib + 4 * g;
-          if (p.dkv_fp32) {
-            *reinterpret_cast<f32x4*>(static_cast<float*>(x ? p.dv : p.dk) + at) = cacc;
-          } else {
+      for (int ip = 0; ip < 4; ++ip) {
+        f32x4 c[2];   // dX^T[in 16 (2 ip + j) + 4 g + i][key]
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int ib = 2 * ip + j;
+          c[j] = mfma_bf16(wa[ib][0], lo0, f32x4{0.f, 0.f, 0.f, 0.f});
+          c[j] = mfma_bf16(wa[ib][0], h0, c[j]);
+          c[j] = mfma_bf16(wa[ib][1], lo1, c[j]);
+          c[j] = mfma_bf16(wa[ib][1], h1, c[j]);
+        }
+        if (p.dkv_fp32) {
+          if (key < key_hi)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              *reinterpret_cast<f32x4*>(static_cast<float*>(x ? p.dv : p.dk) + at + 16 * (2 * ip + j) + 4 * g) = c[j];
+        } else {
+          // One lane-row swap per dword leaves lane g with inputs 32 ip + 16 (g & 1) + 8 (g >> 1) .. +7:
+          // 16 bytes a lane and 64 contiguous bytes a key row per store, where 8-byte pieces gave 32.
+          typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+          typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+          u32x2 pc[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
             bf16x4 v;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = (bf16)cacc[i];
-            *reinterpret_cast<bf16x4*>(static_cast<bf16*>(x ? p.dv : p.dk) + at) = v;
+            for (int i = 0; i < 4; ++i) v[i] = (bf16)c[j][i];
+            pc[j] = __builtin_bit_cast(u32x2, v);
           }
+          u32x4 v;
+#pragma unroll
+          for (int w2 = 0; w2 < 2; ++w2) {
+            const auto r = __builtin_amdgcn_permlane16_swap(pc[0][w2], pc[1][w2], false, false);
+            v[w2] = r[0];
+            v[2 + w2] = r[1];
+          }
+          if (key < key_hi)
+            *reinterpret_cast<u32x4*>(static_cast<bf16*>(x ? p.dv : p.dk) + at + 32 * ip + 16 * (g & 1) + 8 * (g >> 1)) = v;
         }
       }
     }
@@ -799,14 +822,21 @@ __global__ void __launch_bounds__(256) otf_bwd_wreduce_kernel(OtfBwdParams p) {
   const int np = p.B * p.n_sc;
   const float* part = p.wpart + ((size_t)x * p.H + h) * (size_t)np * (kIn * kLat) + e;
   float acc = 0.f;
-  for (int j = 0; j < np; ++j) acc += part[(size_t)j * (kIn * kLat)];
+  for (int j = 0; j < np; j += 8) {   // eight partials in flight, added in order
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = part[(size_t)min(j + q, np - 1) * (kIn * kLat)];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (j + q < np) acc += v[q];
+  }
   const int64_t at = h * p.dw_sh + (e / kLat) * p.dw_si + (e % kLat);
   if (p.dw_fp32) static_cast<float*>(x ? p.dwv : p.dwk)[at] = acc;
   else static_cast<bf16*>(x ? p.dwv : p.dwk)[at] = (bf16)acc;
 }
 
 struct OtfBwdPlan {
-  int Sqp, Skp, n_sc;
+  int Sqp, Skp, chunk, n_sc;
   size_t off_lse2, off_nd, off_klat, off_vlat, off_dx, off_wpart, off_wt, off_bmax, off_gmax, bytes;
 };
 
@@ -814,7 +844,12 @@ OtfBwdPlan make_otf_plan(int64_t B, int64_t H, int64_t Sq, int64_t Sk) {
   OtfBwdPlan pl = {};
   pl.Sqp = (int)((Sq + kRowBlk - 1) / kRowBlk * kRowBlk);
   pl.Skp = (int)((Sk + kKeyBlk - 1) / kKeyBlk * kKeyBlk);
-  pl.n_sc = (int)((Sk + kChunk - 1) / kChunk);
+  // Weight-gradient chunks: 1024 keys, fewer while that leaves workgroups for less than two per CU (a
+  // chunk walks its 64-key blocks serially; each costs a 32 KB partial).  1 x 32 heads x 777 keys:
+  // 26.3 us in one chunk per head and tensor, 13.8 us in seven.
+  pl.chunk = kMaxChunk;
+  while (pl.chunk > kMinChunk && 2 * B * H * ((Sk + pl.chunk - 1) / pl.chunk) < 2 * (int64_t)device_cu_count()) pl.chunk /= 2;
+  pl.n_sc = (int)((Sk + pl.chunk - 1) / pl.chunk);
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   const size_t rows = (size_t)B * H * pl.Sqp, keys = (size_t)B * H * pl.Skp;
   size_t o = 0;
@@ -921,7 +956,7 @@ extern "C" int dmla_bwd_onthefly(const void* q, const void* k, const void* v, co
   p.dw_sh = dw_sh; p.dw_si = dw_si;
   p.B = (int)B; p.H = (int)H; p.Sq = (int)Sq; p.Sk = (int)Sk;
   p.causal = causal ? 1 : 0;
-  p.Sqp = pl.Sqp; p.Skp = pl.Skp; p.n_sc = pl.n_sc;
+  p.Sqp = pl.Sqp; p.Skp = pl.Skp; p.chunk = pl.chunk; p.n_sc = pl.n_sc;
   p.scale = softmax_scale;
   p.scale_log2 = softmax_scale * kLog2e;
   char* ws = static_cast<char*>(workspace);

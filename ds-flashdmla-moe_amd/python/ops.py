@@ -554,7 +554,7 @@ class FlashDMLAOnTheFly(torch.autograd.Function):
 
     Saves q, k, v, wk, wv, o and the row statistics m, l; backward(do) returns the gradients
     of q, k, v, wk and wv (flash_dmla_bwd_onthefly; the weight gradients are summed in fp32 and
-    cast to the weights' dtype by autograd).
+    rounded to the weights' dtype).
     """
 
     @staticmethod
@@ -569,7 +569,7 @@ class FlashDMLAOnTheFly(torch.autograd.Function):
     def backward(ctx, do):
         q, k, v, wk, wv, o, m, l = ctx.saved_tensors
         dq, dk, dv, dwk, dwv = flash_dmla_bwd_onthefly(q, k, v, wk, wv, o, do.contiguous(), m, l,
-                                                       ctx.softmax_scale, ctx.causal)
+                                                       ctx.softmax_scale, ctx.causal, dw_dtype=wk.dtype)
         return dq, dk, dv, dwk, dwv, None, None
 
 
