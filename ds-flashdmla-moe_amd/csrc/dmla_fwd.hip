@@ -159,7 +159,7 @@ struct InlinePlan {
   int fr[kInlinePlanB];        // first range
   int sb[kInlinePlanB + 1];    // first partial slot
   int ctx[kInlinePlanB];       // context length, clamped to the block table
-  int rs[kInlinePlanR + 1];    // range starts
+  int rs[kInlinePlanR + 1];    // range starts; with up to 64 sequences their weighted starts instead
   int tmp[kWaves];             // scan scratch
 };
 constexpr int kDecodeLdsBytes = kLdsBytes + (int)sizeof(InlinePlan);
@@ -465,9 +465,11 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
   // ---- Q through LDS, with the first key tile in flight beside it ---------------------------
   // Chunk k of the staging area is 16-byte chunk k % 73 of row k / 73 (chunk 72 is the row's
   // padding and re-reads chunk 0); rows past the last one re-read row 0 of the item.
+  // Only the 16-row blocks that hold rows are staged; the others' operands are read from block 0.
+  const int q_blocks = (min(kRowsPerWG, nrows - row0) + 15) >> 4;
   auto stage_q = [&]() {
     const unsigned qbase = lds_base + kQOffset;
-    for (int i = wave; i * 64 < kQChunks; i += kWaves) {
+    for (int i = wave; i * 64 < q_blocks * (16 * kQRowBytes / 16); i += kWaves) {
       const int k = i * 64 + lane;
       const int rl = k / (kQRowBytes / 16), ch = k - rl * (kQRowBytes / 16);
       const int rq = row0 + rl;
@@ -516,7 +518,8 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
 #pragma unroll
     for (int c = 0; c < kKcHalf; ++c)
       qreg[qg][c] = lds_read_b128(reinterpret_cast<const DMLA_LDS bf16x8*>(
-          lds + kQOffset + (32 * pair + 16 * qg + l16) * kQRowBytes + (kHalf * (kDqk / 2) + 32 * c + 8 * g) * 2));
+          lds + kQOffset + ((2 * pair + qg < q_blocks ? 32 * pair + 16 * qg : 0) + l16) * kQRowBytes +
+          (kHalf * (kDqk / 2) + 32 * c + 8 * g) * 2));
   __syncthreads();   // Q is read out before the tile copies below reuse its LDS
 
   if (tile_begin < tile_end) {
@@ -813,6 +816,117 @@ __device__ __forceinline__ int wg_exclusive_scan(int v, DMLA_LDS int* tmp, int& 
   return before + x - v;
 }
 
+// Inclusive prefix sum over the wave (DPP row shifts, then row broadcasts: no LDS round trips).
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+struct RangeSpan {
+  int t0, t1, first_b;   // the range's tiles (concatenated tile space) and the sequence of the first
+};
+
+// The decode plan of up to 64 sequences: every wave computes it with one sequence per lane (prefix sums
+// in registers, 32-bit arithmetic: the weighted total is below 2^32), finds its range's ends by a
+// ballot, and wave 0 leaves the per-sequence values in LDS.  One barrier.  The general builder below,
+// with its scans through LDS, 64-bit divisions and one thread placing all ranges of its sequence,
+// took 6.3 us of the 15.6 us the kernel ran at one sequence of 5000 tokens; with this one the call went
+// from 28.0 to 23.5 us there, and from 113.1 to 111.1 us at 64 sequences x 128 heads.  The last
+// workgroup (whose range is the last, never longer than the others) stores the plan for the combine.
+__device__ __forceinline__ RangeSpan build_small_plan(const MqaParams& p, DMLA_LDS InlinePlan* ip, int r) {
+  const int lane = fresh_lane_id();
+  const int wave = uniform(threadIdx.x >> 6);
+  const int B = p.B;
+  const unsigned R = (unsigned)p.n_ranges;
+  int ctx = 0;
+  if (lane < B) ctx = min(max(p.seqlens[lane], 0), p.max_pages * kPage);
+  const int nt = (ctx + kTileN - 1) / kTileN;
+  const int incl = wave_inclusive_scan(nt);
+  const int tp = incl - nt;
+  const int total = __builtin_amdgcn_readlane(incl, 63);
+  const uint64_t nonempty = __ballot(nt > 0);
+  const int nb = __popcll(nonempty & ((1ull << lane) - 1));
+  const unsigned weighted = (unsigned)total + kSegCost * (unsigned)__popcll(nonempty);
+  const unsigned W = uniform((int)max(1u, (weighted + R - 1) / R));
+  const unsigned ws = (unsigned)(tp + kSegCost * nb), we = ws + kSegCost + nt;
+  const unsigned w1 = (unsigned)(tp + kSegCost * (nb + 1));
+  const int fr = nt > 0 ? (int)(w1 / W) : 0;
+  const int ns = nt > 0 ? (int)((w1 + nt - 1) / W) - fr + 1 : 0;
+  const int sincl = wave_inclusive_scan(ns);
+  const int sb = sincl - ns;
+  if (wave == 0) {
+    if (lane < B) {
+      ip->tp[lane] = tp;
+      ip->ns[lane] = ns;
+      ip->fr[lane] = fr;
+      ip->sb[lane] = sb;
+      ip->ctx[lane] = ctx;
+      ip->rs[lane] = (int)ws;
+    }
+    if (lane == 0) {
+      ip->tp[B] = total;
+      ip->sb[B] = __builtin_amdgcn_readlane(sincl, 63);
+    }
+  }
+  // Start of the range at weighted position pos: the sequence holding it, at its first tile while
+  // pos is among its virtual tiles.  Ranges past the weighted total are empty.
+  auto start = [&](unsigned pos, int& b) {
+    b = B - 1;
+    if (pos >= weighted) return total;
+    b = (int)__builtin_ctzll(__ballot(nt > 0 && ws <= pos && pos < we));
+    const int off = (int)(pos - (unsigned)__builtin_amdgcn_readlane((int)ws, b)) - kSegCost;
+    return __builtin_amdgcn_readlane(tp, b) + max(0, off);
+  };
+  RangeSpan sp;
+  int unused;
+  sp.t0 = start((unsigned)min(r, (int)R) * W, sp.first_b);
+  sp.t1 = start((unsigned)min(r + 1, (int)R) * W, unused);
+  __syncthreads();
+  if (blockIdx.x == gridDim.x - 1 && p.plan_out != nullptr) {
+    int32_t* plan = p.plan_out;
+    int32_t* tile_prefix = plan + kPlanHeader;
+    int32_t* split_base = tile_prefix + B + 1;
+    int32_t* num_splits = split_base + B + 1;
+    int32_t* first_range = num_splits + B;
+    int32_t* range_start = first_range + B;
+    int32_t* range_first_b = range_start + R + 1;
+    const int tid = threadIdx.x;
+    if (tid <= B) {
+      tile_prefix[tid] = ip->tp[tid];
+      split_base[tid] = ip->sb[tid];
+    }
+    if (tid < B) {
+      num_splits[tid] = ip->ns[tid];
+      first_range[tid] = ip->fr[tid];
+    }
+    for (int i = tid; i <= (int)R; i += kThreads) {
+      const unsigned pos = (unsigned)i * W;
+      int t = total, lo = B - 1;
+      if (pos < weighted) {   // the last sequence whose weighted start is at or before pos
+        lo = 0;
+        int hi = B - 1;
+        while (lo < hi) {
+          const int mid = (lo + hi + 1) / 2;
+          if ((unsigned)ip->rs[mid] <= pos) lo = mid; else hi = mid - 1;
+        }
+        t = ip->tp[lo] + max(0, (int)(pos - (unsigned)ip->rs[lo]) - kSegCost);
+      }
+      range_start[i] = t;
+      if (i < (int)R) range_first_b[i] = lo;
+    }
+    if (tid == 0) {
+      plan[0] = B; plan[1] = (int)R; plan[2] = (int)W; plan[3] = total; plan[4] = ip->sb[B]; plan[5] = kSegCost;
+      plan[6] = plan[7] = 0;
+    }
+  }
+  return sp;
+}
+
 // The decode plan built by a workgroup in LDS: the arithmetic of decode_plan_kernel with one
 // sequence and one range per thread.  Workgroup 0 also stores it in the plan layout, where
 // the combine reads the split counts and bases.
@@ -926,7 +1040,10 @@ __global__ __launch_bounds__(kThreads, 1) void mqa_fwd_kernel(MqaParams p) {
     const int r = (id / (8 * p.head_groups)) * 8 + id % 8;
     const bool inl = p.plan_inline != 0;
     DMLA_LDS InlinePlan* ip = reinterpret_cast<DMLA_LDS InlinePlan*>(lds + kLdsBytes);
-    if (inl) build_inline_plan(p, ip);   // every workgroup, before any early exit
+    const bool small = inl && p.B <= 64;
+    RangeSpan span = {};
+    if (small) span = build_small_plan(p, ip, r);   // every workgroup, before any early exit
+    else if (inl) build_inline_plan(p, ip);
     if (r >= p.n_ranges) return;
     const int32_t* plan = p.plan;
     const int32_t* tile_prefix = plan + kPlanHeader;
@@ -936,10 +1053,10 @@ __global__ __launch_bounds__(kThreads, 1) void mqa_fwd_kernel(MqaParams p) {
     const int32_t* range_start = first_range + p.B;
     const int32_t* range_first_b = range_start + p.n_ranges + 1;
     auto tp_of = [&](int i) { return inl ? ip->tp[i] : tile_prefix[i]; };
-    const int t0 = inl ? ip->rs[r] : range_start[r];
-    const int t1 = inl ? ip->rs[r + 1] : range_start[r + 1];
+    const int t0 = uniform(small ? span.t0 : inl ? ip->rs[r] : range_start[r]);
+    const int t1 = uniform(small ? span.t1 : inl ? ip->rs[r + 1] : range_start[r + 1]);
     if (t0 >= t1) return;
-    const int first_b = inl ? ip->rfb[r] : range_first_b[r];
+    const int first_b = uniform(small ? span.first_b : inl ? ip->rfb[r] : range_first_b[r]);
     const MqaParams* params = (const MqaParams*)(__builtin_amdgcn_kernarg_segment_ptr());
     for (int bseq = first_b; bseq < p.B; ++bseq) {
       const int tb = tp_of(bseq);

@@ -252,3 +252,33 @@ def test_decode_one_very_long_context(gpu, lens):
     plan = ops.flash_dmla_decode_plan(sl.to(gpu), 128, table.shape[1]).cpu().tolist()
     assert max(R.plan_segment_pages(plan, lens)) <= 128
     _check(gpu, q, pool, table, sl, oracle_device="gpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [16, 128])
+@pytest.mark.parametrize("lens", [
+    [5000], [1], [0, 0, 33],
+    [(37 * b * b) % 700 for b in range(64)],    # one sequence per lane of a wave: the last batch of the register plan
+    [(37 * b * b) % 700 for b in range(65)],    # one more: the plan through LDS scans
+    [0] * 63 + [9000],
+])
+def test_decode_stored_plan_on_both_sides_of_a_wave(gpu, lens, H):
+    """The plan a decode call leaves in its workspace equals the plan kernel's for batches around 64
+    sequences, and the call decodes like the same call with that plan handed in."""
+    from python import _lib
+    q, pool, table, sl = (t.to(gpu) for t in _paged(lens, H, seed=110 + len(lens)))
+    B, max_pages = len(lens), table.shape[1]
+    plan = ops.flash_dmla_decode_plan(sl, H, max_pages)
+    ws_bytes = int(_lib.lib().dmla_decode_workspace_bytes(B, H, 512, max_pages))
+    ws = torch.full((ws_bytes,), 0x5A, dtype=torch.uint8, device=gpu)
+    o = torch.empty((B, H, 512), dtype=torch.bfloat16, device=gpu)
+    _lib.call("dmla_decode_paged", q.data_ptr(), pool.data_ptr(), table.data_ptr(), sl.data_ptr(), o.data_ptr(), None,
+              B, H, 576, 512, 64, pool.shape[0], max_pages, q.stride(0), q.stride(1), pool.stride(0), pool.stride(1),
+              table.stride(0), o.stride(0), o.stride(1), SCALE, ws.data_ptr(), ws_bytes,
+              torch.cuda.current_stream().cuda_stream)
+    n = 8 + 4 * B + 2 + 2 * int(plan[1]) + 1
+    assert torch.equal(ws[:4 * n].view(torch.int32), plan[:n])
+    planned = ops.flash_dmla_decode_paged(q, pool, table, sl, 512, SCALE, plan=plan)
+    assert torch.equal(o, planned)
+    o_ref, _ = R.dmla_decode_paged(q.float().cpu(), pool.float().cpu(), table.cpu(), sl.cpu(), 512, SCALE)
+    assert_out_close(o, o_ref)
