@@ -112,6 +112,7 @@ struct MqaParams {
   int max_pages;
   int head_groups;     // ceil(H / 64)
   int n_ranges;        // R of the decode plan
+  int round_ranges;    // ranges that run at once (decode_round)
   const int32_t* plan; // decode plan (see decode_plan_kernel); unused when plan_inline
   int plan_inline;     // every workgroup builds the plan in LDS (B <= kInlinePlanB, R <= kInlinePlanR)
   int32_t* plan_out;   // with plan_inline: workgroup 0 stores the plan here (the combine reads it)
@@ -137,8 +138,9 @@ struct Work {
 // prologue and epilogue (loading Q and the first tile, writing the output) of about
 // kSegCost tiles, so the ranges are equal in the weighted space where each nonempty sequence
 // is preceded by kSegCost virtual tiles: range r starts at weighted position r W with
-// W = ceil(weighted total / R), moved to the sequence's first tile when it falls among the
-// virtual ones.  The work per workgroup is then about the same whatever the context lengths.
+// W = plan_width(weighted total), moved to the sequence's first tile when it falls among the
+// virtual ones; ranges past the weighted total are empty.  The work per workgroup is then about the
+// same whatever the context lengths.
 // Layout (int32): header[8] = {B, R, W, total tiles, total splits, kSegCost, 0, 0}, then
 // tile_prefix[B + 1], split_base[B + 1] (first partial slot of each sequence), num_splits[B],
 // first_range[B], range_start[R + 1] (first tile of each range, in the concatenated tile
@@ -146,6 +148,21 @@ struct Work {
 constexpr int kPlanHeader = 8;
 constexpr int kSegCost = 10;   // per-segment cost in tiles: a launch timeline fits 0.92 us per tile + 9.2 us per segment
 constexpr int kMaxSegTiles = 2 * kMaxSegPages - 2;   // a segment's pages fit its page registers
+// Width of a range.  The chip runs P ranges at once (decode_round), and R may be more, because it is
+// sized on the host for full block tables with no segment past its page registers.  Cutting the work
+// in R > P ranges costs a second round of workgroups for the few past P.  So the ranges are cut for
+// whole rounds: one where no segment can be too long (tables of up to kMaxSegPages pages), else as
+// many as the actual contexts need; the ranges left over are empty.  Measured (R ranges -> whole
+// rounds, us per call): 128 sequences of 1024..8192 tokens x 128 heads 292 -> 191 (R = 135, P = 128),
+// 256 x 128 heads 485 -> 393, 256 x 16 heads 358 -> 256 (R = 269, P = 256), 40 of 4000..32768 x 128
+// heads 305 -> 238, 600 of 16..4096 x 32 heads (plan kernel) 362 -> 302; R = P 111 -> 111.
+template <typename T>
+__device__ __forceinline__ T plan_width(T weighted, T R, T P, int max_pages) {
+  const T per_round = P * (T)kMaxSegTiles;
+  const T rounds = max_pages <= kMaxSegPages ? (T)1 : max((T)1, (T)((weighted + per_round - 1) / per_round));
+  const T cut = min(R, P * rounds);
+  return max((T)1, (T)((weighted + cut - 1) / cut));
+}
 __host__ __device__ inline int64_t plan_ints(int64_t B, int64_t R) { return kPlanHeader + 4 * B + 2 + 2 * R + 1; }
 // Inline plan: the decode kernel builds the plan itself, in LDS past the pipeline's area, when
 // the batch and the range count fit (the common serving case); the standalone plan kernel and
@@ -852,7 +869,7 @@ __device__ __forceinline__ RangeSpan build_small_plan(const MqaParams& p, DMLA_L
   const uint64_t nonempty = __ballot(nt > 0);
   const int nb = __popcll(nonempty & ((1ull << lane) - 1));
   const unsigned weighted = (unsigned)total + kSegCost * (unsigned)__popcll(nonempty);
-  const unsigned W = uniform((int)max(1u, (weighted + R - 1) / R));
+  const unsigned W = uniform((int)plan_width<unsigned>(weighted, R, (unsigned)p.round_ranges, p.max_pages));
   const unsigned ws = (unsigned)(tp + kSegCost * nb), we = ws + kSegCost + nt;
   const unsigned w1 = (unsigned)(tp + kSegCost * (nb + 1));
   const int fr = nt > 0 ? (int)(w1 / W) : 0;
@@ -943,7 +960,7 @@ __device__ __forceinline__ void build_inline_plan(const MqaParams& p, DMLA_LDS I
   const int tpb = wg_exclusive_scan(nt, ip->tmp, total);
   const int nb = wg_exclusive_scan(nt > 0 ? 1 : 0, ip->tmp, nonempty);
   const int64_t weighted = (int64_t)total + (int64_t)kSegCost * nonempty;
-  const int W = (int)max<int64_t>(1, (weighted + R - 1) / R);
+  const int W = (int)plan_width<int64_t>(weighted, R, p.round_ranges, p.max_pages);
   // Each nonempty sequence owns the weighted positions [ws, ws + kSegCost + nt): its kSegCost
   // virtual tiles, then its tiles.  The ranges starting there (r W in that span) start at its
   // first tile or at the tile under r W -- the value the plan kernel's search over sequences
@@ -1187,8 +1204,8 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(MqaParams p) {
 constexpr int kPlanLds = 4096;
 constexpr int kPlanThreads = 256;   // four waves: the scans and barriers stay short
 constexpr int kPlanWaves = kPlanThreads / 64;
-__global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(const int32_t* seqlens, int B, int R, int max_pages,
-                                                           int32_t* plan) {
+__global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(const int32_t* seqlens, int B, int R, int P,
+                                                           int max_pages, int32_t* plan) {
   __shared__ int scan[kPlanThreads];
   __shared__ int l_tp[kPlanLds], l_ne[kPlanLds], l_rs[kPlanLds];
   int32_t* tile_prefix = plan + kPlanHeader;
@@ -1252,7 +1269,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(const int32_t
   const int total = carry;
   if (tid == 0) { tile_prefix[B] = total; if (lds_b) l_tp[B] = total; }
   const int64_t weighted = (int64_t)total + (int64_t)kSegCost * ncarry;
-  const int W = (int)max<int64_t>(1, (weighted + R - 1) / R);
+  const int W = (int)plan_width<int64_t>(weighted, R, P, max_pages);
   __threadfence_block();
   __syncthreads();
   // Range starts: weighted position r W -> the sequence holding it (last b whose weighted start
@@ -1320,18 +1337,22 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(const int32_t
   }
 }
 
-// Ranges of a decode plan: one workgroup per range and head group fills the CUs; more ranges
-// when the widest batch would overflow a segment's page cache.  A segment spans at most W
-// tiles, W = ceil(weighted / R), and the weighted total is at most B max_pages 2 + kSegCost B
-// (every sequence full and nonempty), so R >= that bound / kMaxSegTiles keeps W <= kMaxSegTiles
-// and every segment within kMaxSegPages pages (a segment may start on the second tile of a page).
-int64_t decode_ranges(int64_t B, int64_t H, int64_t max_pages) {
+// Ranges the chip runs at once: one workgroup per range and head group fills the CUs.
+int64_t decode_round(int64_t H) {
   const int64_t hg = (H + kRowsPerWG - 1) / kRowsPerWG;
   int64_t r = device_cu_count() / hg;
   if (r >= 8) r -= r % 8;
+  return std::max<int64_t>(r, 1);
+}
+// Ranges a decode plan has room for: a round, or more when the widest batch would overflow a
+// segment's page cache.  A segment spans at most W tiles and the weighted total is at most
+// B max_pages 2 + kSegCost B (every sequence full and nonempty), so with R >= that bound /
+// kMaxSegTiles, plan_width can keep W <= kMaxSegTiles and every segment within kMaxSegPages pages
+// (a segment may start on the second tile of a page).
+int64_t decode_ranges(int64_t B, int64_t H, int64_t max_pages) {
   const int64_t weighted_max = B * max_pages * (kPage / kTileN) + (int64_t)kSegCost * B;
   const int64_t cap = (weighted_max + kMaxSegTiles - 1) / kMaxSegTiles;
-  return std::max<int64_t>(std::max<int64_t>(r, cap), 1);
+  return std::max<int64_t>(decode_round(H), cap);
 }
 
 }  // namespace
@@ -1552,7 +1573,7 @@ extern "C" int dmla_decode_plan(const int32_t* cache_seqlens, int64_t B, int64_t
                 (long long)plan_bytes);
   const int64_t R = decode_ranges(B, H, max_pages_per_seq);
   hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(kPlanThreads), 0, (hipStream_t)stream, cache_seqlens, (int)B, (int)R,
-                     (int)max_pages_per_seq, plan);
+                     (int)decode_round(H), (int)max_pages_per_seq, plan);
   return check_launch("dmla_decode_plan");
 }
 
@@ -1625,12 +1646,16 @@ int decode_launch(const void* q, const void* kv_pool, const int32_t* block_table
   p.max_pages = (int)max_pages_per_seq;
   p.head_groups = (int)((H + kRowsPerWG - 1) / kRowsPerWG);
   p.n_ranges = (int)decode_ranges(B, H, max_pages_per_seq);
+  p.round_ranges = (int)decode_round(H);
   p.plan = plan_out != nullptr ? nullptr : plan;
   p.plan_inline = plan_out != nullptr ? 1 : 0;
   p.plan_out = plan_out;
   p.part_o = static_cast<bf16*>(workspace);
   p.part_lse = reinterpret_cast<float*>(p.part_o + slots * H * kDv);
-  const int64_t grid = ((int64_t)(p.n_ranges + 7) / 8) * 8 * p.head_groups;
+  // A plan built by the kernel has no more ranges than one round where the tables are short
+  // (plan_width); a plan handed in is taken as it is.
+  const int64_t live = plan_out != nullptr && max_pages_per_seq <= kMaxSegPages ? p.round_ranges : p.n_ranges;
+  const int64_t grid = (live + 7) / 8 * 8 * p.head_groups;
   if (grid > 0x7fffffff) return fail(DMLA_ERR_UNSUPPORTED, "dmla_decode_paged: grid too large");
   hipLaunchKernelGGL(mqa_fwd_kernel<true>, dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
   int rc = check_launch("dmla_decode_paged");

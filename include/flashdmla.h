@@ -170,9 +170,10 @@ int dmla_decode_paged_noalloc(const void* q, const void* kv_pool, const int32_t*
  * more if a range's pages could exceed 128), each processed by one workgroup per head group.
  * Every piece of a sequence inside a range is one split of it (a segment of the workgroup's
  * work); sequences with several splits are merged by the LSE combine.  A segment has a fixed
- * cost (loading Q and its first tile, writing its output) of about 16 tiles, so the ranges are
- * equal in a weighted space where each nonempty sequence is preceded by 16 virtual tiles:
- * every workgroup gets about the same work whatever the lengths.  plan (int32,
+ * cost (loading Q and its first tile, writing its output) of about 10 tiles, so the ranges are
+ * equal in a weighted space where each nonempty sequence is preceded by 10 virtual tiles:
+ * every workgroup gets about the same work whatever the lengths.  Where R is more than the ranges
+ * that run at once, W is that of whole rounds of them and the ranges left over are empty.  plan (int32,
  * dmla_decode_plan_bytes bytes):
  *   [0..7]   B, R, W (weighted tiles per range), total tiles, total splits, segment cost, 0, 0
  *   then     tile_prefix[B + 1], split_base[B + 1], num_splits[B], first_range[B],

@@ -187,14 +187,16 @@ def dmla_decode_paged(q: Tensor, kv_pool: Tensor, block_table: Tensor, cache_seq
 
 
 def decode_plan(cache_seqlens, n_ranges: int, max_pages: int, page_size: int = 64, tile: int = 32,
-                seg_cost: int = 10):
+                seg_cost: int = 10, per_round: int = 0, max_seg_pages: int = 128):
     """The decode tile-scheduler plan for R = n_ranges (no reference counterpart).
 
     The 32-token tiles of all sequences, in order, are cut into R ranges that are equal in a
     weighted space where every nonempty sequence is preceded by seg_cost virtual tiles (the
     fixed cost of a segment): range r starts at weighted position r*W, W = ceil(weighted/R),
     which maps to the tile at that position, or to the sequence's first tile when the position
-    is among its virtual tiles.  Returns the int32 list header[8] + tile_prefix[B+1] +
+    is among its virtual tiles.  With per_round (the ranges that run at once) below R, W is that
+    of whole rounds: of one where tables have at most max_seg_pages pages, else of as many as keep
+    W within 2*max_seg_pages - 2 tiles (at most R ranges).  Returns the int32 list header[8] + tile_prefix[B+1] +
     split_base[B+1] + num_splits[B] + first_range[B] + range_start[R+1] + range_first_b[R]
     with the layout of include/flashdmla.h."""
     B, R = len(cache_seqlens), n_ranges
@@ -208,7 +210,11 @@ def decode_plan(cache_seqlens, n_ranges: int, max_pages: int, page_size: int = 6
         wstart.append(tp[b] + seg_cost * ne)
         ne += tiles[b] > 0
     weighted = total + seg_cost * ne
-    W = max(1, -(-weighted // R))
+    cut = R
+    if per_round:
+        rounds = 1 if max_pages <= max_seg_pages else max(1, -(-weighted // (per_round * (2 * max_seg_pages - 2))))
+        cut = min(R, per_round * rounds)
+    W = max(1, -(-weighted // cut))
     rs = []
     for r in range(R):
         pos = r * W

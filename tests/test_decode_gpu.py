@@ -282,3 +282,44 @@ def test_decode_stored_plan_on_both_sides_of_a_wave(gpu, lens, H):
     assert torch.equal(o, planned)
     o_ref, _ = R.dmla_decode_paged(q.float().cpu(), pool.float().cpu(), table.cpu(), sl.cpu(), 512, SCALE)
     assert_out_close(o, o_ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,lens,max_pages", [
+    (128, [(37 * b * b) % 300 for b in range(140)], 128),           # more ranges than a round, all in one
+    (2048, [700 * b for b in range(12)], 128),                      # the same in the register plan
+    (2048, [700 * b for b in range(12)], 129),                      # rounds counted: tables past a segment's pages
+    (2048, [36000, 30000, 0, 5000], 600),                           # two rounds of ranges needed
+    (2048, [36000] + [0, 500, 64] * 30, 600),                       # the plan through LDS scans
+    (128, [(37 * b * b) % 100 for b in range(520)], 128),           # the plan kernel's batches
+])
+def test_decode_plan_with_more_ranges_than_a_round(gpu, H, lens, max_pages):
+    """Where a plan has room for more ranges than run at once, it fills whole rounds: the plan equals
+    the oracle's, no segment is too long, and the plan a decode call builds itself is the same."""
+    from python import _lib
+    q, pool, table, sl = (t.to(gpu) for t in _paged(lens, H, seed=130 + len(lens)))
+    B, width = len(lens), table.shape[1]
+    wide = torch.zeros((B, max_pages), dtype=torch.int32, device=gpu)
+    wide[:, :width] = table
+    hg = -(-H // 64)
+    per_round = torch.cuda.get_device_properties(0).multi_processor_count // hg
+    per_round = max(per_round - per_round % 8 if per_round >= 8 else per_round, 1)
+    plan = ops.flash_dmla_decode_plan(sl, H, max_pages)
+    got = plan.cpu().tolist()
+    assert got[1] > per_round
+    ref = R.decode_plan(lens, got[1], max_pages, per_round=per_round)
+    assert got[:len(ref)] == ref
+    assert max(R.plan_segment_pages(got, lens)) <= 128
+    ws_bytes = int(_lib.lib().dmla_decode_workspace_bytes(B, H, 512, max_pages))
+    ws = torch.full((ws_bytes,), 0x5A, dtype=torch.uint8, device=gpu)
+    o = torch.empty((B, H, 512), dtype=torch.bfloat16, device=gpu)
+    _lib.call("dmla_decode_paged", q.data_ptr(), pool.data_ptr(), wide.data_ptr(), sl.data_ptr(), o.data_ptr(), None,
+              B, H, 576, 512, 64, pool.shape[0], max_pages, q.stride(0), q.stride(1), pool.stride(0), pool.stride(1),
+              wide.stride(0), o.stride(0), o.stride(1), SCALE, ws.data_ptr(), ws_bytes,
+              torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert ws.view(torch.int32)[:len(ref)].cpu().tolist() == ref
+    o2, _ = ops.flash_dmla_decode_paged(q, pool, wide, sl, 512, SCALE, return_lse=True, plan=plan)
+    assert torch.equal(o, o2)
+    o_ref, _ = R.dmla_decode_paged(q[:, :64].cpu().float(), pool.cpu().float(), table.cpu(), sl.cpu(), 512, SCALE)
+    assert_out_close(o[:, :64], o_ref)
