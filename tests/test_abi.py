@@ -60,6 +60,31 @@ def test_fwd_argument_errors():
     assert _lib.lib().dmla_last_error() == b""
 
 
+def test_fwd_ws_errors_are_those_of_the_plain_forward():
+    """The entry point with a workspace refuses what the plain one refuses, whatever the workspace;
+    unsupported and empty problems need none."""
+    P = ctypes.c_void_p
+    lib = _lib.lib()
+
+    def call(B=1, Sq=512, dqk=576, dv=512, scale=0.07, q=1 << 20, m=None, ws=None, ws_bytes=0):
+        return lib.dmla_fwd_cache_latent_ws(
+            P(q), P(1 << 20), P(1 << 20), P(m), P(None), B, 16, Sq, 8192, dqk, dv,
+            16 * 512 * 576, 512 * 576, 576, 8192 * 576, 576, 16 * 512 * 512, 512 * 512, 512,
+            scale, 1, P(ws), ws_bytes, None)
+
+    for ws, n in ((None, 0), (1 << 20, 1 << 40)):
+        assert call(q=None, ws=ws, ws_bytes=n) == _lib.DMLA_ERR_INVALID_ARG
+        assert call(q=(1 << 20) + 2, ws=ws, ws_bytes=n) == _lib.DMLA_ERR_INVALID_ARG
+        assert call(m=1 << 20, ws=ws, ws_bytes=n) == _lib.DMLA_ERR_INVALID_ARG
+        assert call(scale=-1.0, ws=ws, ws_bytes=n) == _lib.DMLA_ERR_INVALID_ARG
+        assert call(dqk=64, dv=32, ws=ws, ws_bytes=n) == _lib.DMLA_ERR_UNSUPPORTED
+        assert call(B=0, ws=ws, ws_bytes=n) == _lib.DMLA_OK
+        assert call(Sq=0, ws=ws, ws_bytes=n) == _lib.DMLA_OK
+    assert lib.dmla_fwd_workspace_bytes(1, 16, 512, 8192, 64, 32, 1) == 0
+    assert lib.dmla_fwd_workspace_bytes(0, 16, 512, 8192, 576, 512, 1) == 0
+    assert lib.dmla_fwd_workspace_bytes(4, 16, 2048, 2048, 576, 512, 1) == 0   # enough row tiles
+
+
 def test_decode_argument_errors():
     P = ctypes.c_void_p
     lib = _lib.lib()
