@@ -27,11 +27,11 @@
 // Softmax: in log2 units against a per-row reference max m_ref that only moves when a tile's
 // max exceeds it by more than kSlack (p <= 2^kSlack in between); moving it rescales O and l.  The exact running max is tracked beside it for the m / l outputs, which
 // follow the cache-latent forward's convention (natural-log units).
-#include <algorithm>
 #include <type_traits>
 
 #include "dmla_common.h"
 #include "dmla_host.h"
+#include "dmla_rules.h"
 
 namespace dmla {
 namespace {
@@ -701,30 +701,6 @@ __global__ void __launch_bounds__(kOtfThreads, 1) otf_fwd_short_kernel(OtfParams
 
 using namespace dmla;
 
-// Query rows per workgroup: 512 (otf_fwd_kernel) or 256 / 128 (otf_fwd_short_kernel).  A workgroup of
-// n key tiles takes about fixed_us + n tile_us, measured at 1 x 32 heads x 500 and 777 rows
-// (one workgroup per CU) and 2 x 32 x 4096 (all CUs busy): larger tiles cost less per row (the
-// projection is shared by more of them), smaller ones occupy more CUs and end sooner.  The estimate
-// is the larger of the chip's share of the work and the longest workgroup; the smallest wins.
-// Measured sides: 1 x 32 x 500 takes 34.4 / 20.4 / 16.9 us and 2 x 32 x 4096 234 / 291 / 401 us with
-// 512 / 256 / 128 rows.
-static int otf_tile(int64_t BH, int64_t Sq, int64_t Sk, int causal) {
-  static constexpr struct { int rows; double tile_us, fixed_us; } shapes[] = {
-      {kOtfRows, 2.9, 12.0}, {256, 2.0, 5.0}, {128, 1.5, 4.2}};
-  int best = 0;
-  double best_us = 0;
-  for (const auto& s : shapes) {
-    const double n_wg = (double)((Sq + s.rows - 1) / s.rows) * (double)BH;
-    // keys seen by a row tile: all of them, or on average those up to the middle tile's last row
-    const double rows = (double)std::min<int64_t>(Sq, s.rows);
-    const double keys = causal ? std::min((double)Sk, std::max(0.0, (double)(Sk - Sq) + 0.5 * ((double)Sq + rows))) : (double)Sk;
-    const double us = std::max(n_wg / device_cu_count() * (s.fixed_us + s.tile_us * keys / kOtfKeys),
-                               s.fixed_us + s.tile_us * (double)Sk / kOtfKeys);
-    if (best == 0 || us < best_us) { best = s.rows; best_us = us; }
-  }
-  return best;
-}
-
 extern "C" int dmla_fwd_onthefly(const void* q, const void* k, const void* v, const void* wk, const void* wv,
                                  void* o, float* m, float* l, int64_t B, int64_t H, int64_t Sq, int64_t Sk,
                                  int64_t d_in, int64_t d_lat, int64_t q_sb, int64_t q_sh, int64_t q_ss,
@@ -769,7 +745,7 @@ extern "C" int dmla_fwd_onthefly(const void* q, const void* k, const void* v, co
   p.causal = causal ? 1 : 0;
   p.scale_log2 = softmax_scale * kLog2e;
   p.o_rows16 = mult8(o_sb) && mult8(o_sh) && mult8(o_ss);
-  const int rows = otf_tile(B * H, Sq, Sk, p.causal);
+  const int rows = otf_rows(device_cu_count(), B * H, Sq, Sk, p.causal);
   p.n_qt = (int)((Sq + rows - 1) / rows);
   const int64_t grid = (int64_t)p.n_qt * B * H;
   if (grid > 0x7fffffff) return fail(DMLA_ERR_UNSUPPORTED, "dmla_fwd_onthefly: grid too large");

@@ -92,22 +92,25 @@ def test_otf_strided_views(gpu):
     [
         # 128 rows per workgroup, two waves per row block: rows that see keys of one half only, a
         # ragged last tile in either half, several row tiles
-        (1, 2, 20, 20, True),
-        (1, 2, 129, 95, False),
+        (1, 3, 130, 165, True),
+        (1, 2, 300, 357, False),
         (1, 3, 257, 129, True),
         (2, 32, 700, 700, True),
-        # 256 rows per workgroup
-        (16, 32, 130, 130, True),
-        (16, 32, 257, 600, False),
         (3, 32, 513, 700, True),
+        # 256 rows per workgroup
+        (1, 2, 20, 20, True),
+        (1, 2, 129, 95, False),
+        (16, 32, 130, 130, True),
         # 512 rows per workgroup
+        (16, 32, 257, 600, False),
         (16, 32, 257, 257, True),
         (16, 16, 300, 300, False),
         (16, 32, 500, 1000, True),
     ],
 )
 def test_otf_row_tiles(gpu, B, H, Sq, Sk, causal):
-    """The three workgroup shapes the launcher's estimate picks among, at their edges."""
+    """The three workgroup shapes the launcher's estimate picks among, at their edges
+    (tests/test_rules.py holds the shape that runs each size)."""
     _check(gpu, B, H, Sq, Sk, causal, seed=Sq + Sk, ref_device="gpu")
 
 
