@@ -28,12 +28,12 @@
 //    stays below 2^kHeadroom, so O is never rescaled.  Scores climbing past that headroom
 //    trigger a recomputation of the row tile from a higher reference.
 #include <algorithm>
-#include <cmath>
 #include <mutex>
 #include <type_traits>
 
 #include "dmla_common.h"
 #include "dmla_host.h"
+#include "dmla_rules.h"
 
 namespace dmla {
 namespace {
@@ -87,8 +87,6 @@ __device__ __forceinline__ void iteration_schedule() {
   __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 }
 
-constexpr int kMaxParts = 32;   // key ranges of a split prefill row tile
-
 struct MqaParams {
   const bf16* q;
   const bf16* kv;
@@ -118,12 +116,12 @@ struct MqaParams {
   int32_t* plan_out;   // with plan_inline: workgroup 0 stores the plan here (the combine reads it)
   bf16* part_o;        // [slots, H, 512] normalised partial outputs, rounded to bf16
   float* part_lse;     // [slots, H]
-  // prefill with split key ranges (PrefillSplit; slot = workgroup id)
+  // prefill with split key ranges (PrefillSplit)
   float* part_o32;     // [slots, 64 rows, 512] normalised partial outputs
   float2* part_ml;     // [slots, 64 rows] (max in log2 units, row sum relative to it)
   int n_layers;
-  int first_rt[kMaxParts];        // first row tile with more than j parts
-  int layer_base[kMaxParts + 1];  // row tiles (of one batch element) in the layers before j
+  int first_rt[kPrefillMaxParts];        // first row tile with more than j parts
+  int layer_base[kPrefillMaxParts + 1];  // row tiles (of one batch element) in the layers before j
 };
 
 struct Work {
@@ -1116,6 +1114,11 @@ __device__ __forceinline__ int prefill_parts(const MqaParams& p, int rt) {
   for (int j = 1; j < p.n_layers; ++j) n += rt >= p.first_rt[j] ? 1 : 0;
   return n;
 }
+// Slot of part j of a row tile with several parts: the layers in order, without the row tiles of layer
+// 0 that have one part (n_row_tiles - first_rt[1] have more).
+__device__ __forceinline__ int prefill_slot(const MqaParams& p, int b, int j, int rt) {
+  return (p.layer_base[j] - (j > 0 ? p.first_rt[1] : 0) + p.n_row_tiles - 1 - rt) * p.B + b;
+}
 
 __global__ __launch_bounds__(kThreads, 1) void mqa_fwd_split_kernel(MqaParams p) {
   __shared__ __attribute__((aligned(1024))) char smem[kLdsBytes];
@@ -1133,7 +1136,7 @@ __global__ __launch_bounds__(kThreads, 1) void mqa_fwd_split_kernel(MqaParams p)
   wk.nsplit = prefill_parts(p, rt);
   wk.tile_begin = (int)((int64_t)n * j / wk.nsplit);
   wk.tile_end = (int)((int64_t)n * (j + 1) / wk.nsplit);
-  wk.slot = (int)blockIdx.x;
+  wk.slot = prefill_slot(p, wk.b, j, rt);   // not used with one part
   const MqaParams* params = (const MqaParams*)(__builtin_amdgcn_kernarg_segment_ptr());
   if (((wave >> 1) & 1) == 0) mqa_fwd_body<false, 0, false, true>(p, params, wk, lds, wave, lane);
   else mqa_fwd_body<false, 1, false, true>(p, params, wk, lds, wave, lane);
@@ -1151,19 +1154,19 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(MqaParams p) {
   const int r = rt * kRowsPerWG + rl;
   if (r >= p.H * p.Sq) return;
   const int n = prefill_parts(p, rt);
-  auto slot = [&](int j) { return (int64_t)(p.layer_base[j] + p.n_row_tiles - 1 - rt) * p.B + b; };
+  auto slot = [&](int j) { return (int64_t)prefill_slot(p, b, j, rt); };
   // the parts' (m, l) sit in lanes 0 .. n - 1
   const int64_t own = slot(min(lane, n - 1));
   float2 ml = p.part_ml[own * kRowsPerWG + rl];
   if (lane >= n) ml = make_float2(kNegInf, 0.f);
   float mx = ml.x;
 #pragma unroll
-  for (int o = 1; o < kMaxParts; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  for (int o = 1; o < kPrefillMaxParts; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   mx = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mx)));
   const float w = mx == kNegInf ? 0.f : ml.y * fast_exp2(ml.x - mx);
   float wsum = w;
 #pragma unroll
-  for (int o = 1; o < kMaxParts; o <<= 1) wsum += __shfl_xor(wsum, o, 64);
+  for (int o = 1; o < kPrefillMaxParts; o <<= 1) wsum += __shfl_xor(wsum, o, 64);
   wsum = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wsum)));
   f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
   for (int j0 = 0; j0 < n; j0 += 4) {
@@ -1363,82 +1366,7 @@ using namespace dmla;
 namespace dmla {
 namespace {
 
-struct PrefillSplit {
-  int n_layers;                    // most parts of a row tile; 1: no split
-  int first_rt[kMaxParts];
-  int layer_base[kMaxParts + 1];
-  int64_t slots() const { return layer_base[n_layers]; }   // per batch element
-};
-
-int64_t prefill_tiles_host(int64_t H, int64_t Sq, int64_t Sk, int causal, int64_t rt) {
-  const int64_t last_pos = (std::min<int64_t>((rt + 1) * kRowsPerWG, H * Sq) - 1) / H;
-  const int64_t kend = causal ? std::min(Sk, last_pos + 1 + (Sk - Sq)) : Sk;
-  return (std::max<int64_t>(kend, 0) + kTileN - 1) / kTileN;
-}
-
-// Whether and how to split the key ranges of a prefill.  A workgroup of n key tiles takes about
-// kFixedUs + n kTileUs (measured: prologue and epilogue, and the tile loop), a merge kMergeUs,
-// kMergePartUs per part of a row and 4 KB of traffic per row and part at ~4 TB/s.  Unsplit, some CU
-// runs j + 1 workgroups at least as long as the (j CUs)-th longest.  Only calls with at most four
-// row tiles per CU are considered: past that the grid balances itself.  Measured sides (16 heads,
-// causal): 512 of 8192 positions 201 us unsplit, 135 in two parts, 156 in three; 4 of 8000 192 us
-// unsplit, 32 in 16 parts; 1024 of 1024 (row tiles of 1 to 32 tiles, one per CU) 32 us unsplit, 43
-// with the longest cut in two.
-constexpr double kFixedUs = 5.5, kTileUs = 0.85, kMergeUs = 4.0, kMergePartUs = 0.4;
-PrefillSplit prefill_split(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int causal) {
-  PrefillSplit sp = {};
-  const int64_t n_rt = (H * Sq + kRowsPerWG - 1) / kRowsPerWG, cus = device_cu_count();
-  sp.n_layers = 1;
-  sp.layer_base[1] = (int)n_rt;
-  if (n_rt * B > 4 * cus) return sp;
-  auto tiles = [&](int64_t rt) { return prefill_tiles_host(H, Sq, Sk, causal, rt); };
-  const int64_t nmax = tiles(n_rt - 1);
-  // at most 64 row tiles stand for all of them
-  const int64_t step = (n_rt + 63) / 64;
-  double total = 0;
-  int64_t samples = 0;
-  for (int64_t rt = n_rt - 1; rt >= 0; rt -= step, ++samples) total += (double)tiles(rt);
-  const double mean = total / (double)samples;
-  double best = 0;
-  for (int64_t j = 0; j * cus < n_rt * B; ++j)
-    best = std::max(best, (double)(j + 1) * (kFixedUs + kTileUs * (double)tiles(n_rt - 1 - j * cus / B)));
-  best = 0.92 * std::max(best, (double)(n_rt * B) * (kFixedUs + kTileUs * mean) / (double)cus);
-  int64_t best_t = 0;
-  static constexpr int kTry[] = {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
-  for (int s : kTry) {
-    const int64_t t = (nmax + s - 1) / s;
-    if (t < 4) break;
-    double parts = 0, merged = 0;
-    for (int64_t rt = n_rt - 1; rt >= 0; rt -= step) {
-      const int64_t np = std::max<int64_t>(1, (tiles(rt) + t - 1) / t);
-      parts += (double)np;
-      if (np > 1) merged += (double)np;
-    }
-    const double scale = (double)n_rt * (double)B / (double)samples;
-    const double wgs = parts * scale;
-    const double rounds = std::max(1.0, std::ceil(wgs / (double)cus - 0.01));
-    const double part_us = kFixedUs + kTileUs * mean * (double)samples / parts;
-    const double us = std::max(kFixedUs + kTileUs * (double)t, rounds * part_us) + kMergeUs + kMergePartUs * (double)s +
-                      merged * scale * kRowsPerWG * 4096.0 / 4e6;
-    if (us < best) { best = us; best_t = t; }
-  }
-  if (best_t == 0) return sp;
-  sp.n_layers = (int)std::min<int64_t>((nmax + best_t - 1) / best_t, kMaxParts);
-  int64_t base = 0;
-  for (int j = 0; j < sp.n_layers; ++j) {
-    int64_t lo = 0, hi = n_rt;   // first row tile with more than j parts: tiles > j best_t (all have part 0)
-    while (j > 0 && lo < hi) {
-      const int64_t mid = (lo + hi) / 2;
-      if (tiles(mid) > j * best_t) hi = mid; else lo = mid + 1;
-    }
-    sp.first_rt[j] = (int)lo;
-    sp.layer_base[j] = (int)base;
-    base += n_rt - lo;
-  }
-  sp.layer_base[sp.n_layers] = (int)base;
-  return sp;
-}
-
+static_assert(kRowsPerWG == kPrefillRows && kTileN == kPrefillKeys, "the split rule counts these tiles");
 int64_t prefill_slot_bytes() { return kRowsPerWG * (int64_t)(kDv * 4 + 8); }
 
 // Both prefill entry points; a workspace of the split's size (dmla_fwd_workspace_bytes) lets it run.
@@ -1486,7 +1414,7 @@ int fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, float*
   const int64_t grid = (int64_t)p.n_row_tiles * B;
   if (grid > 0x7fffffff) return fail(DMLA_ERR_UNSUPPORTED, "dmla_fwd_cache_latent: grid too large");
   PrefillSplit sp = {};
-  if (split) sp = prefill_split(B, H, Sq, Sk, p.causal);
+  if (split) sp = prefill_split(device_cu_count(), B, H, Sq, Sk, p.causal);
   if (sp.n_layers <= 1) {
     hipLaunchKernelGGL(mqa_fwd_kernel<false>, dim3((unsigned)grid), dim3(kThreads), 0, stream, p);
     return check_launch("dmla_fwd_cache_latent");
@@ -1501,7 +1429,7 @@ int fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, float*
   p.n_layers = sp.n_layers;
   for (int j = 0; j < sp.n_layers; ++j) p.first_rt[j] = sp.first_rt[j];
   for (int j = 0; j <= sp.n_layers; ++j) p.layer_base[j] = sp.layer_base[j];
-  hipLaunchKernelGGL(mqa_fwd_split_kernel, dim3((unsigned)slots), dim3(kThreads), 0, stream, p);
+  hipLaunchKernelGGL(mqa_fwd_split_kernel, dim3((unsigned)(sp.workgroups() * B)), dim3(kThreads), 0, stream, p);
   const int64_t merged = (p.n_row_tiles - sp.first_rt[1]) * B;
   hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)(16 * merged)), dim3(256), 0, stream, p);
   return check_launch("dmla_fwd_cache_latent_ws");
@@ -1526,7 +1454,7 @@ extern "C" int64_t dmla_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, in
   if (B > ((int64_t)1 << 30) || H > ((int64_t)1 << 30) || Sq > ((int64_t)1 << 30) || H * Sq > ((int64_t)1 << 30) ||
       Sk > ((int64_t)1 << 30))
     return 0;
-  const PrefillSplit sp = prefill_split(B, H, Sq, Sk, causal ? 1 : 0);
+  const PrefillSplit sp = prefill_split(device_cu_count(), B, H, Sq, Sk, causal ? 1 : 0);
   return sp.n_layers > 1 ? sp.slots() * B * prefill_slot_bytes() : 0;
 }
 

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 
 namespace dmla {
 
@@ -97,6 +98,97 @@ inline int otf_rows(int cus, int64_t BH, int64_t Sq, int64_t Sk, int causal) {
     }
   }
   return best;
+}
+
+// ---- cache-latent prefill: key ranges split over workgroups -----------------------------------
+constexpr int kPrefillRows = 64, kPrefillKeys = 32;   // rows of a row tile, keys of a key tile
+constexpr int kPrefillMaxParts = 32;                  // key ranges of a row tile
+
+struct PrefillSplit {
+  int n_layers;                           // most parts of a row tile; 1: no split
+  int first_rt[kPrefillMaxParts];         // layer j holds part j of the row tiles from first_rt[j] on
+  int layer_base[kPrefillMaxParts + 1];   // row tiles (of one batch element) in the layers before j
+  int64_t workgroups() const { return layer_base[n_layers]; }   // per batch element
+  // Partials, per batch element: the row tiles with one part (those before first_rt[1]) write none.
+  int64_t slots() const { return n_layers > 1 ? layer_base[n_layers] - first_rt[1] : 0; }
+};
+
+inline int64_t prefill_key_tiles(int64_t H, int64_t Sq, int64_t Sk, int causal, int64_t rt) {
+  const int64_t last_pos = (std::min<int64_t>((rt + 1) * kPrefillRows, H * Sq) - 1) / H;
+  const int64_t kend = causal ? std::min(Sk, last_pos + 1 + (Sk - Sq)) : Sk;
+  return (std::max<int64_t>(kend, 0) + kPrefillKeys - 1) / kPrefillKeys;
+}
+
+// Whether and how to split the key ranges of a prefill.  A workgroup of n key tiles takes about
+// kFixedUs + n kTileUs (measured: prologue and epilogue, and the tile loop), a merge kMergeUs,
+// kMergePartUs per part of a row and 4 KB of traffic per row and part at ~4 TB/s.  Unsplit, some CU
+// runs j + 1 workgroups at least as long as the (j CUs)-th longest.  Only calls with at most four
+// row tiles per CU are considered: past that the grid balances itself.  Measured sides (16 heads,
+// causal): 512 of 8192 positions 201 us unsplit, 135 in two parts, 156 in three; 4 of 8000 192 us
+// unsplit, 32 in 16 parts; 1024 of 1024 (row tiles of 1 to 32 tiles, one per CU) 32 us unsplit, 43
+// with the longest cut in two.  A split has at most kSplitWgsPerCu workgroups per CU, which caps the
+// workspace at 16 x 132 KB per CU (539 MB on 256 CUs; 5 x 5 heads, 2047 of 137187 positions took 842 MB in
+// 6400 workgroups).  More of them hardly even anything out: by the estimate the bound costs nothing up
+// to 8192 keys, and that call takes 13.9 ms in 4000 against 14.1 in 6400, 15.6 in 1600 and 18.1 unsplit.
+constexpr double kFixedUs = 5.5, kTileUs = 0.85, kMergeUs = 4.0, kMergePartUs = 0.4;
+constexpr int64_t kSplitWgsPerCu = 16;
+inline PrefillSplit prefill_split(int64_t cus, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int causal) {
+  PrefillSplit sp = {};
+  const int64_t n_rt = (H * Sq + kPrefillRows - 1) / kPrefillRows;
+  sp.n_layers = 1;
+  sp.layer_base[1] = (int)n_rt;
+  if (n_rt * B > 4 * cus) return sp;
+  auto tiles = [&](int64_t rt) { return prefill_key_tiles(H, Sq, Sk, causal, rt); };
+  const int64_t nmax = tiles(n_rt - 1);
+  // at most 64 row tiles stand for all of them
+  const int64_t step = (n_rt + 63) / 64;
+  double total = 0;
+  int64_t samples = 0;
+  for (int64_t rt = n_rt - 1; rt >= 0; rt -= step, ++samples) total += (double)tiles(rt);
+  const double mean = total / (double)samples;
+  double best = 0;
+  for (int64_t j = 0; j * cus < n_rt * B; ++j)
+    best = std::max(best, (double)(j + 1) * (kFixedUs + kTileUs * (double)tiles(n_rt - 1 - j * cus / B)));
+  best = 0.92 * std::max(best, (double)(n_rt * B) * (kFixedUs + kTileUs * mean) / (double)cus);
+  int64_t best_t = 0;
+  static constexpr int kTry[] = {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
+  for (int s : kTry) {
+    const int64_t t = (nmax + s - 1) / s;
+    if (t < 4) break;
+    double parts = 0, merged = 0;
+    for (int64_t rt = n_rt - 1; rt >= 0; rt -= step) {
+      const int64_t np = std::max<int64_t>(1, (tiles(rt) + t - 1) / t);
+      parts += (double)np;
+      if (np > 1) merged += (double)np;
+    }
+    const double scale = (double)n_rt * (double)B / (double)samples;
+    const double wgs = parts * scale;
+    if (wgs > (double)(kSplitWgsPerCu * cus)) break;
+    const double rounds = std::max(1.0, std::ceil(wgs / (double)cus - 0.01));
+    const double part_us = kFixedUs + kTileUs * mean * (double)samples / parts;
+    const double us = std::max(kFixedUs + kTileUs * (double)t, rounds * part_us) + kMergeUs + kMergePartUs * (double)s +
+                      merged * scale * kPrefillRows * 4096.0 / 4e6;
+    if (us < best) { best = us; best_t = t; }
+  }
+  if (best_t == 0) return sp;
+  const int64_t most = kSplitWgsPerCu * cus / B;   // workgroups per batch element
+  do {
+    sp.n_layers = (int)std::min<int64_t>((nmax + best_t - 1) / best_t, kPrefillMaxParts);
+    int64_t base = 0;
+    for (int j = 0; j < sp.n_layers; ++j) {
+      int64_t lo = 0, hi = n_rt;   // first row tile with more than j parts: tiles > j best_t (all have part 0)
+      while (j > 0 && lo < hi) {
+        const int64_t mid = (lo + hi) / 2;
+        if (tiles(mid) > j * best_t) hi = mid; else lo = mid + 1;
+      }
+      sp.first_rt[j] = (int)lo;
+      sp.layer_base[j] = (int)base;
+      base += n_rt - lo;
+    }
+    sp.layer_base[sp.n_layers] = (int)base;
+    best_t += (best_t + 15) / 16;
+  } while (sp.workgroups() > most && sp.n_layers > 1);   // where the samples stood for too few parts
+  return sp;
 }
 
 }  // namespace dmla

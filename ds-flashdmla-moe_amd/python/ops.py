@@ -136,7 +136,8 @@ def flash_dmla_fwd(
     if return_stats:
         m = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
         l = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
-    # Calls that leave CUs idle split their key ranges through a workspace (0 bytes: no split).
+    # Calls whose row tiles leave CUs idle, at first or in the last round, split their key ranges through
+    # a workspace (0 bytes: no split).
     ws_bytes = int(_lib.lib().dmla_fwd_workspace_bytes(B, H, Sq, Sk, Dqk, d_v, 1 if causal else 0))
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device) if ws_bytes else None
     _lib.call(

@@ -68,12 +68,13 @@ int dmla_fwd_cache_latent(const void* q, const void* k_lat, void* o, float* m, f
                           float softmax_scale, int causal, dmla_stream_t stream);
 
 /*
- * dmla_fwd_cache_latent with a workspace, for calls whose row tiles leave CUs idle (a chunk of a long
- * prompt, a few short prompts): the keys of a row tile are cut over several workgroups, whose fp32
- * partials and row statistics a second kernel merges.  Same arguments, results and checks;
- * dmla_fwd_workspace_bytes gives the bytes needed on the current device (16-byte aligned device
- * memory, contents ignored), 0 where the call would not be split and runs as
- * dmla_fwd_cache_latent does (the workspace may then be NULL).
+ * dmla_fwd_cache_latent with a workspace, for calls of at most four 64-row tiles per CU whose row
+ * tiles leave CUs idle, at first or in the last round (a chunk of a long prompt, a few short prompts):
+ * the keys of a row tile are cut over several workgroups, whose fp32 partials and row statistics a
+ * second kernel merges.  Same arguments, results and checks; dmla_fwd_workspace_bytes gives the bytes
+ * needed on the current device (16-byte aligned device memory, contents ignored; at most 16 x 131584
+ * per CU, 539 MB on 256 CUs), 0 where the call would not be split and runs as dmla_fwd_cache_latent
+ * does (the workspace may then be NULL).
  */
 int64_t dmla_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t d_qk,
                                  int64_t d_v, int causal);

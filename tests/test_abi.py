@@ -85,6 +85,15 @@ def test_fwd_ws_errors_are_those_of_the_plain_forward():
     assert lib.dmla_fwd_workspace_bytes(4, 16, 2048, 2048, 576, 512, 1) == 0   # enough row tiles
 
 
+def test_fwd_workspace_is_bounded():
+    """At most sixteen workgroups per CU (256 where there is no GPU) hold a partial of 64 rows of 512 fp32
+    values and two statistics, however long the context; a row tile with one part holds none."""
+    lib = _lib.lib()
+    slot = 64 * (512 * 4 + 8)
+    for shape in ((5, 5, 2047, 137187), (1, 16, 512, 1 << 20), (16, 1, 64, 1 << 20), (1, 1, 700, 700)):
+        assert 0 < lib.dmla_fwd_workspace_bytes(*shape, 576, 512, 1) <= 16 * 256 * slot
+
+
 def test_decode_argument_errors():
     P = ctypes.c_void_p
     lib = _lib.lib()

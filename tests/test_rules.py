@@ -30,6 +30,14 @@ int main() {
       for (const auto& s : dmla::kOtfShapes)
         std::printf(" %.9g", dmla::otf_estimate_us(s, (int)cus, bh, sq, sk, (int)causal));
       std::printf("\n");
+    } else {
+      long cus, b, h, sq, sk, causal;
+      if (std::scanf("%ld %ld %ld %ld %ld %ld", &cus, &b, &h, &sq, &sk, &causal) != 6) return 1;
+      const dmla::PrefillSplit sp = dmla::prefill_split(cus, b, h, sq, sk, (int)causal);
+      std::printf("%d %ld %ld", sp.n_layers, (long)sp.workgroups(), (long)sp.slots());
+      for (int j = 0; j < sp.n_layers; ++j) std::printf(" %d", sp.first_rt[j]);
+      for (int j = 0; j <= sp.n_layers; ++j) std::printf(" %d", sp.layer_base[j]);
+      std::printf("\n");
     }
   }
 }
@@ -134,3 +142,36 @@ def test_otf_rows_over_all_sizes_and_devices(ask):
              (1 << 31, 1, 1, True), (7, 300, 20, True), (1, 1 << 24, 5, True), (1024, 1, 1 << 30, False), (3, 40000, 40000, True)]
     for cus in (1, 32, 64, 256, 304, 1000):
         assert all(r in (128, 256, 512) for r, _ in _otf(ask, sizes, cus))
+
+
+def test_prefill_split_layout_and_bound(ask):
+    """Every part of a row tile with several parts has a slot of its own, row tiles with one part have
+    none, and the workgroups (with them the workspace) are bounded by sixteen per CU."""
+    rng = random.Random(4)
+    sizes = [(5, 5, 2047, 137187, 1), (1, 1, 700, 700, 1), (1, 16, 512, 8192, 1), (16, 128, 3, 41, 1), (1, 8, 6148, 8182, 0)]
+    while len(sizes) < 400:
+        b, h, sq = rng.randint(1, 16), 1 << rng.randint(0, 7), int(2 ** rng.uniform(0, 13))
+        sizes.append((b, h, sq, sq if rng.random() < 0.3 else int(2 ** rng.uniform(0, 18)), rng.randint(0, 1)))
+    splits = ragged = 0
+    for cus in (256, 64):
+        out = ask([f"prefill {cus} {b} {h} {sq} {sk} {c}" for b, h, sq, sk, c in sizes])
+        for (b, h, sq, sk, c), line in zip(sizes, out):
+            n, wgs, slots, *rest = map(int, line)
+            n_rt = -(-h * sq // 64)
+            if n == 1:
+                assert (wgs, slots) == (n_rt, 0)
+                continue
+            splits += 1
+            first, base = rest[:n], rest[n:]
+            assert wgs * b <= 16 * cus and first == sorted(first) and first[0] == 0 and base[0] == 0
+            used = []
+            for rt in range(n_rt):
+                parts = sum(rt >= f for f in first)
+                tiles = -(-(min(sk, (min((rt + 1) * 64, h * sq) - 1) // h + 1 + sk - sq) if c else sk) // 32)
+                assert 1 <= parts <= max(tiles, 1)
+                if parts > 1:
+                    used += [base[j] - (first[1] if j else 0) + n_rt - 1 - rt for j in range(parts)]
+                ragged += parts == 1
+            assert sorted(used) == list(range(slots)), (b, h, sq, sk, c)
+            assert wgs == slots + first[1]
+    assert splits > 100 and ragged > 0
