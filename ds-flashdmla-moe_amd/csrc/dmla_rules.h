@@ -15,12 +15,14 @@ struct OtfShape {
   double tile_us;     // of CUs with a workgroup
   double busy_us;
 };
-// Measured at 340 sizes (B * H of 8..512, 16..8192 rows and keys): the estimate below is within 4 % of each
+// Measured at 510 sizes (B * H of 8..512, 16..8192 rows and keys): the estimate below is within 4 % of each
 // shape's time on average.
 constexpr OtfShape kOtfShapes[] = {{512, 6.0, 2.75, 0.4}, {256, 3.7, 1.7, 0.3}, {128, 4.6, 1.25, 0.2}};
 constexpr double kOtfTileBytes = 2 * 64 * 128 * 2;   // the raw K and V rows of a 64-key tile
-constexpr double kOtfCacheBytes = 256e6;             // K and V past this come from HBM again for each row tile
-constexpr double kOtfHbmBytesPerUs = 4.2e6;          // at this rate
+// K and V of more than kOtfCacheBytes come from HBM again, at kOtfHbmBytesPerUs, for each set of row
+// tiles of a head that run at once.
+constexpr double kOtfCacheBytes = 256e6;
+constexpr double kOtfHbmBytesPerUs = 4.8e6;
 
 // Key tiles (64 keys) of row tile qt of `rows` query rows.
 inline int64_t otf_key_tiles(int rows, int64_t qt, int64_t Sq, int64_t Sk, int causal) {
@@ -75,23 +77,27 @@ inline double otf_estimate_us(const OtfShape& s, int cus, int64_t BH, int64_t Sq
   } else {
     for (int64_t j = 0; j < 64 && (double)j * cus < n; ++j) us = std::max(us, (double)(j + 1) * len(nq - 1 - j * cus / BH));
   }
-  if ((double)BH * (double)Sk * 512.0 > kOtfCacheBytes)
-    us = std::max(us, n * (mean - s.fixed_us) / tile_us * kOtfTileBytes / kOtfHbmBytesPerUs);
+  if ((double)BH * (double)Sk * 512.0 > kOtfCacheBytes) {
+    const double together = std::max(1.0, std::min((double)nq, cus / (double)BH));
+    const double hbm_us = n * (mean - s.fixed_us) / tile_us * kOtfTileBytes / together / kOtfHbmBytesPerUs;
+    us = std::sqrt(us * us + hbm_us * hbm_us);   // neither hides the other whole
+  }
   return us;
 }
 
 // Query rows per workgroup: larger tiles cost less per row (the projection is shared by more of
-// them), smaller ones occupy more CUs and end sooner.  The smallest estimate wins, the larger tile on a tie.
+// them), smaller ones occupy more CUs and end sooner.  The smallest estimate wins, the larger tile on a
+// tie; 512 rows keep 5 %, about what the estimates are off.
 // Measured with 512 / 256 / 128 rows: 1 x 32 x 500 causal 34.4 / 20.4 / 16.9 us, 2 x 32 x 4096 causal
 // 234 / 291 / 401; non-causal 1 x 32 x 2100 109 / 133 / 150 and 1 x 32 x 1100 58 / 38 / 57 (288 workgroups
 // of 128 rows on 256 CUs).  Counting rounds as fractions took the 256 rows at 1 x 32 x 2100 and the 128 at
-// 1 x 32 x 1100: over 340 sizes it was up to 1.5x off the best shape and 1.3x slower than 512 rows; this
-// estimate is 1.06x off at most and 0.2 % on average.
+// 1 x 32 x 1100: over 510 sizes it was up to 1.5x off the best shape and 1.3x slower than 512 rows; this
+// choice is 4.5 % off at most, 0.2 % on average, and at most 2.6 % slower than 512 rows.
 inline int otf_rows(int cus, int64_t BH, int64_t Sq, int64_t Sk, int causal) {
   int best = 0;
   double best_us = 0;
   for (const OtfShape& s : kOtfShapes) {
-    const double us = otf_estimate_us(s, cus, BH, Sq, Sk, causal);
+    const double us = (s.rows == 512 ? 0.95 : 1.0) * otf_estimate_us(s, cus, BH, Sq, Sk, causal);
     if (best == 0 || us < best_us) {
       best = s.rows;
       best_us = us;

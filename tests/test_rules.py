@@ -79,6 +79,7 @@ def _otf(ask, sizes, cus=256):
         (24, 3639, 8036, False, 512),
         (160, 463, 463, False, 512),
         (144, 2028, 4254, True, 512),
+        (96, 2048, 8056, True, 512),     # K and V past the last cache: more row tiles, more HBM traffic
         (32, 1100, 1100, False, 256),    # 160 workgroups; 288 of 128 rows would run two rounds
         (64, 513, 513, False, 256),
         # The listed sizes of the forward's measurements keep their shapes.
@@ -112,11 +113,12 @@ def test_otf_estimate_is_the_schedule(ask):
     while len(sizes) < 300:
         bh, sq = rng.randint(8, 300), rng.randint(1, 6000)
         sk = sq if rng.random() < 0.5 else rng.randint(1, 8192)
-        if bh * sk * 512 <= 256e6:   # past that the estimate may be the HBM time instead
+        if bh * sk * 512 <= 256e6:   # past that the estimate counts HBM traffic too
             sizes.append((bh, sq, sk, rng.random() < 0.5))
     cus = 256
     for (bh, sq, sk, causal), (rows, est) in zip(sizes, _otf(ask, sizes, cus)):
-        assert est[rows] == min(est.values())
+        biased = {r: e * (0.95 if r == 512 else 1.0) for r, e in est.items()}
+        assert biased[rows] == min(biased.values())
         for r, (fixed, tile, busy) in shapes.items():
             nq = -(-sq // r)
             n = nq * bh
