@@ -840,15 +840,20 @@ struct OtfBwdPlan {
   size_t off_lse2, off_nd, off_klat, off_vlat, off_dx, off_wpart, off_wt, off_bmax, off_gmax, bytes;
 };
 
-OtfBwdPlan make_otf_plan(int64_t B, int64_t H, int64_t Sq, int64_t Sk) {
+// Keys per weight-gradient workgroup: 1024, fewer while that leaves workgroups for less than two per CU (a
+// chunk walks its 64-key blocks serially; each costs a 32 KB partial).  1 x 32 heads x 777 keys: 26.3 us
+// in one chunk per head and tensor, 13.8 us in seven.
+int otf_wgrad_chunk(int64_t B, int64_t H, int64_t Sk) {
+  int chunk = kMaxChunk;
+  while (chunk > kMinChunk && 2 * B * H * ((Sk + chunk - 1) / chunk) < 2 * (int64_t)device_cu_count()) chunk /= 2;
+  return chunk;
+}
+
+OtfBwdPlan make_otf_plan(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int chunk) {
   OtfBwdPlan pl = {};
   pl.Sqp = (int)((Sq + kRowBlk - 1) / kRowBlk * kRowBlk);
   pl.Skp = (int)((Sk + kKeyBlk - 1) / kKeyBlk * kKeyBlk);
-  // Weight-gradient chunks: 1024 keys, fewer while that leaves workgroups for less than two per CU (a
-  // chunk walks its 64-key blocks serially; each costs a 32 KB partial).  1 x 32 heads x 777 keys:
-  // 26.3 us in one chunk per head and tensor, 13.8 us in seven.
-  pl.chunk = kMaxChunk;
-  while (pl.chunk > kMinChunk && 2 * B * H * ((Sk + pl.chunk - 1) / pl.chunk) < 2 * (int64_t)device_cu_count()) pl.chunk /= 2;
+  pl.chunk = chunk;
   pl.n_sc = (int)((Sk + pl.chunk - 1) / pl.chunk);
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   const size_t rows = (size_t)B * H * pl.Sqp, keys = (size_t)B * H * pl.Skp;
@@ -878,7 +883,7 @@ extern "C" int64_t dmla_bwd_onthefly_workspace_bytes(int64_t B, int64_t H, int64
                                                      int64_t d_lat) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || d_in != kIn || d_lat != kLat) return 0;
   if (Sq > kOtfBwdMaxSeq || Sk > kOtfBwdMaxSeq) return 0;
-  return (int64_t)make_otf_plan(B, H, Sq, Sk).bytes;
+  return (int64_t)make_otf_plan(B, H, Sq, Sk, otf_wgrad_chunk(B, H, Sk)).bytes;
 }
 
 extern "C" int dmla_bwd_onthefly(const void* q, const void* k, const void* v, const void* wk, const void* wv,
@@ -918,7 +923,10 @@ extern "C" int dmla_bwd_onthefly(const void* q, const void* k, const void* v, co
   if (B == 0 || H == 0) return DMLA_OK;
   if (Sq == 0 || Sk == 0)
     return fail(DMLA_ERR_INVALID_ARG, "dmla_bwd_onthefly: Sq and Sk must be > 0 (zero the gradients instead)");
-  const OtfBwdPlan pl = make_otf_plan(B, H, Sq, Sk);
+  // A workspace below the query's size takes longer chunks (fewer partials), down to that of 1024 keys, the
+  // size that does not depend on the device.
+  OtfBwdPlan pl = make_otf_plan(B, H, Sq, Sk, otf_wgrad_chunk(B, H, Sk));
+  while (workspace_bytes < (int64_t)pl.bytes && pl.chunk < kMaxChunk) pl = make_otf_plan(B, H, Sq, Sk, 2 * pl.chunk);
   if (workspace_bytes < (int64_t)pl.bytes || !workspace)
     return fail(DMLA_ERR_WORKSPACE, "dmla_bwd_onthefly: workspace of %lld bytes needed, got %lld",
                 (long long)pl.bytes, (long long)workspace_bytes);

@@ -238,3 +238,48 @@ def test_otf_bwd_strided_inputs(gpu):
     _, _, _, ref = _run(gpu, (q, k, v, wk, wv, do), True)
     for name, a, b in zip(NAMES, grads, ref):
         assert torch.equal(a, b), f"{name}: strided inputs change the result"
+
+
+def _wgrad_chunk(gpu, B, H, Sk):
+    """Keys per weight-gradient workgroup: 1024, halved down to 128 while that leaves less than two per CU."""
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    chunk = 1024
+    while chunk > 128 and 2 * B * H * -(-Sk // chunk) < 2 * cus:
+        chunk //= 2
+    return chunk
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,Sq,Sk", [(1, 2, 200, 700), (2, 1, 70, 1500)])
+def test_otf_bwd_smaller_workspace(gpu, B, H, Sq, Sk):
+    """The query's workspace holds a partial per chunk of the length that fills the device; one that holds
+    only the partials of 1024-key chunks (its size on any device) runs with those, a byte less is
+    refused.  dq, dk and dv do not depend on the chunks; the weight gradients are the same fp32 sums in
+    another order, Sk terms of at most ~1e2 that add to values of that size: 1e-3 absolute is > 100 ulps."""
+    from python import _lib
+    q, k, v, wk, wv, do = (t.to(gpu) for t in _inputs(B, H, Sq, Sk, seed=Sk))
+    o, m, l = ops.flash_dmla_fwd_onthefly(q, k, v, wk, wv, 0.125, True, return_stats=True)
+    ref = ops.flash_dmla_bwd_onthefly(q, k, v, wk, wv, o, do, m, l, 0.125, True)
+    chunks = -(-Sk // _wgrad_chunk(gpu, B, H, Sk))
+    need = _lib.lib().dmla_bwd_onthefly_workspace_bytes(B, H, Sq, Sk, 128, 64)
+    least = need - 65536 * B * H * (chunks - -(-Sk // 1024))
+    assert least < need
+
+    def call(ws_bytes):
+        out = [torch.full_like(t, float("nan")) for t in ref]
+        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=gpu)
+        P, st = ops._ptr, lambda t: tuple(t.stride())
+        rc = _lib.lib().dmla_bwd_onthefly(
+            *map(P, (q, k, v, wk, wv, o, do, m, l)), *map(P, out), B, H, Sq, Sk, 128, 64, *st(q)[:3], *st(k)[:3],
+            *st(v)[:3], *st(wk)[:2], *st(o)[:3], *st(do)[:3], *st(out[0])[:3], *st(out[1])[:3], *st(out[3])[:2],
+            0, 0, 1, 0.125, 1, P(ws), ws_bytes, ops._stream(q))
+        return rc, out
+
+    assert call(least - 1)[0] == _lib.DMLA_ERR_WORKSPACE
+    for ws_bytes in (least, need - 1):
+        rc, out = call(ws_bytes)
+        assert rc == _lib.DMLA_OK
+        for name, a, b in zip(NAMES[:3], out, ref):
+            assert torch.equal(a, b), name
+        for name, a, b in zip(NAMES[3:], out[3:], ref[3:]):
+            assert (a - b).abs().max().item() <= 1e-3, name
