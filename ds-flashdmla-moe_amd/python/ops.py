@@ -137,18 +137,26 @@ def flash_dmla_fwd(
         m = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
         l = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
     # Calls whose row tiles leave CUs idle, at first or in the last round, split their key ranges through
-    # a workspace (0 bytes: no split).
+    # a workspace (0 bytes: no split); where it does not fit in memory they run unsplit.
     ws_bytes = int(_lib.lib().dmla_fwd_workspace_bytes(B, H, Sq, Sk, Dqk, d_v, 1 if causal else 0))
-    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device) if ws_bytes else None
-    _lib.call(
-        "dmla_fwd_cache_latent_ws",
+    ws = None
+    if ws_bytes:
+        try:
+            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:
+            pass
+    args = (
         _ptr(q), _ptr(k_lat), _ptr(o), _ptr(m), _ptr(l),
         B, H, Sq, Sk, Dqk, d_v,
         q.stride(0), q.stride(1), q.stride(2),
         k_lat.stride(0), k_lat.stride(1),
         o.stride(0), o.stride(1), o.stride(2),
-        _scale(softmax_scale, Dqk), 1 if causal else 0, _ptr(ws), ws_bytes, _stream(q),
+        _scale(softmax_scale, Dqk), 1 if causal else 0,
     )
+    if ws is not None or not ws_bytes:
+        _lib.call("dmla_fwd_cache_latent_ws", *args, _ptr(ws), ws_bytes, _stream(q))
+    else:
+        _lib.call("dmla_fwd_cache_latent", *args, _stream(q))
     return o, m, l
 
 

@@ -136,3 +136,26 @@ def test_fwd_split_key_ranges(gpu, B, H, Sq, Sk, causal, split):
     o_ref, m_ref, l_ref = R.dmla_fwd_cache_latent(q.float(), k2.float(), 512, SCALE, causal)
     assert_stats_close(m, l, m_ref, l_ref)
     assert ((o.float() - o_ref).abs().max() / o_ref.abs().max()).item() <= 1e-2
+
+
+@pytest.mark.gpu
+def test_fwd_without_memory_for_the_workspace(gpu, monkeypatch):
+    """A call that would split its key ranges runs unsplit where the workspace does not fit in memory."""
+    q = seeded((1, 16, 64, 576), 90, 0.5, torch.bfloat16).to(gpu)
+    k = seeded((1, 2000, 576), 91, 0.5, torch.bfloat16).to(gpu)
+    assert ops._lib.lib().dmla_fwd_workspace_bytes(1, 16, 64, 2000, 576, 512, 1) > 0
+    ref = [torch.empty(*s, dtype=t, device=gpu) for s, t in
+           (((1, 16, 64, 512), torch.bfloat16), ((1, 16, 64), torch.float32), ((1, 16, 64), torch.float32))]
+    ops._lib.call("dmla_fwd_cache_latent", *map(ops._ptr, (q, k, *ref)), 1, 16, 64, 2000, 576, 512, *q.stride()[:3],
+                  *k.stride()[:2], *ref[0].stride()[:3], SCALE, 1, ops._stream(q))
+    empty = torch.empty
+
+    def no_workspace(*args, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no memory for the workspace")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_workspace)
+    out = ops.flash_dmla_fwd(q, k, 512, SCALE, True)
+    for a, b in zip(out, ref):
+        assert torch.equal(a, b)
