@@ -142,7 +142,7 @@ __device__ __forceinline__ void combine_pair(const CombineArgs& a, const T* part
 // pair, 1 (four pairs per 256-thread block) or 4.
 template <bool kPlan, int kW>
 __global__ void __launch_bounds__(256) lse_combine_kernel(CombineArgs a) {
-  __shared__ float xch[kW == 1 ? 1 : kW * 64 * 8];
+  __shared__ f32x4 xch[kW == 1 ? 1 : kW * 64 * 2];   // kW rows of up to 512 sums, as 16-byte pieces
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   // 32-bit index math: the launcher checks B * H < 2^31

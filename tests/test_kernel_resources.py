@@ -97,3 +97,21 @@ def test_backward_kernels_keep_occupancy_without_spills(tmp_path, source):
     for name, want in _BWD_OCCUPANCY[source].items():
         assert name in stats, f"{name} not found in {source}"
         assert stats[name][2] >= want, f"{name}: occupancy {stats[name][2]} < {want} ({stats[name][0]} VGPRs)"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is needed")
+@pytest.mark.parametrize("source", ["dmla_bwd.hip", "dmla_cache.hip", "dmla_fwd.hip", "dmla_otf.hip", "dmla_otf_bwd.hip"])
+def test_lds_arrays_are_aligned_for_their_vector_accesses(tmp_path, source):
+    """LDS byte and float arrays are accessed as 16-byte vectors: each one declares that alignment
+    itself, whatever other LDS variables its kernel gets.  (Half and int arrays here are accessed
+    element by element.)"""
+    out = tmp_path / (source + ".ll")
+    flags = [f for f in FLAGS if f != "-S"]
+    run = subprocess.run([HIPCC] + flags + ["-S", "-emit-llvm", "-Xclang", "-disable-llvm-passes",
+                                            os.path.join(CSRC, source), "-o", str(out)],
+                         capture_output=True, text=True, timeout=600)
+    assert run.returncode == 0, run.stderr[-2000:]
+    arrays = re.findall(r"^@(\S+) = .*addrspace\(3\) global \[(\d+) x (i8|float|<\d+ x \w+>)\].*align (\d+)", out.read_text(), re.M)
+    assert arrays, "no LDS array found"
+    for name, _, kind, align in arrays:
+        assert int(align) >= 16, f"{name}: [{kind}] array with alignment {align}"
