@@ -263,3 +263,35 @@ def test_bwd_long_sequence_is_chunked(gpu, monkeypatch):
     assert ws < (512 << 20) + (200 << 20), ws
     q, k, do = _inputs(1, 16, 8192, 8192, seed=5)
     _check(gpu, q, k, do, True, ref_device="gpu", autograd=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "B,H,Sq,Sk,causal",
+    [
+        (1, 1, 33, 400, True),     # four segments a pair; the middle key block, alone in its pair, has two steps
+        (1, 1, 100, 64 * 9, False),
+        (1, 2, 600, 450, True),    # rows without keys, up to 32 segments
+        (2, 16, 391, 391, True),   # segments in several batches of four partials
+    ],
+)
+def test_bwd_segment_reduction(gpu, B, H, Sq, Sk, causal):
+    """dK_lat's sum over the segments of a pair: segment counts around the batches of four, segments
+    without steps (whose partials are not written), segments that meet one key block of the pair only."""
+    q, k, do = _inputs(B, H, Sq, Sk, seed=Sq + Sk)
+    _check(gpu, q, k, do, causal, ref_device="gpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cap", [None, 96 * 1024])
+def test_autograd_dk_is_the_rounded_fp32_gradient(gpu, monkeypatch, cap):
+    """The autograd function takes dk_lat in k_lat's dtype: the fp32 sum rounded once, last, bit for bit
+    what a cast of the fp32 output gives, in one chunk of rows or several."""
+    if cap is not None:
+        monkeypatch.setenv("DMLA_BWD_DS_CAP_BYTES", str(cap))
+    q, k, do = _inputs(2, 4, 300, 300, seed=61)
+    qg, kg = q.to(gpu).requires_grad_(True), k.to(gpu).requires_grad_(True)
+    ops.flash_dmla(qg, kg, 512, SCALE, True).backward(do.to(gpu))
+    _, _, _, dq, dk = _run(gpu, q, k, do, True, dk_dtype=torch.float32)
+    assert kg.grad.dtype == torch.bfloat16 and torch.equal(kg.grad, dk.to(torch.bfloat16))
+    assert torch.equal(qg.grad, dq)

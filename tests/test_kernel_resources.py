@@ -115,3 +115,41 @@ def test_lds_arrays_are_aligned_for_their_vector_accesses(tmp_path, source):
     assert arrays, "no LDS array found"
     for name, _, kind, align in arrays:
         assert int(align) >= 16, f"{name}: [{kind}] array with alignment {align}"
+
+
+def _compile(tmp_path, source):
+    out = tmp_path / (source + ".s")
+    run = subprocess.run([HIPCC] + FLAGS + [os.path.join(CSRC, source), "-o", str(out)],
+                         capture_output=True, text=True, timeout=600)
+    assert run.returncode == 0, run.stderr[-2000:]
+    return out.read_text()
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is needed")
+def test_split_prefill_tile_loop_is_spill_free(tmp_path):
+    """The prefill with split key ranges under the rules of the kernels it shares its body with: no
+    scratch access in a tile iteration, and outside of them only beside the exact-path call."""
+    asm = _compile(tmp_path, "dmla_fwd.hip")
+    start = asm.index("_ZN4dmla12_GLOBAL__N_120mqa_fwd_split_kernelENS0_9MqaParamsE:")
+    ins = [l.strip() for l in asm[start:asm.index(".Lfunc_end", start)].split("\n")]
+    calls = [i for i, l in enumerate(ins) if l.startswith("s_swappc")]
+    assert calls, "the exact-path call is expected in the kernel"
+    tiles = 0
+    for blk in _blocks(ins):
+        if sum(l.startswith("v_mfma") for l in blk) >= 16 and not any(l.startswith("s_swappc") for l in blk):
+            tiles += 1
+            assert not [l for l in blk if l.startswith("scratch_")]
+    assert tiles > 0
+    far = [i for i, l in enumerate(ins) if l.startswith("scratch_") and all(abs(i - c) > 40 for c in calls)]
+    assert len(far) <= 4, f"{len(far)} scratch accesses outside the exact-path call"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc is needed")
+def test_onthefly_forwards_keep_occupancy_without_spills(tmp_path):
+    """One workgroup of eight waves per CU: two waves per SIMD, so at most 256 registers and no scratch."""
+    asm = _compile(tmp_path, "dmla_otf.hip")
+    for name in ("14otf_fwd_kernelE", "20otf_fwd_short_kernelILi1EE", "20otf_fwd_short_kernelILi2EE"):
+        rest = asm[re.search(r"^_ZN4dmla\S*%s\S*:" % name, asm, re.M).end():]
+        vgprs, scratch, occupancy = (int(re.search(r"; %s: (\d+)" % key, rest).group(1))
+                                     for key in ("NumVgprs", "ScratchSize", "Occupancy"))
+        assert scratch == 0 and occupancy >= 2, f"{name}: {scratch} bytes of scratch, occupancy {occupancy}, {vgprs} VGPRs"

@@ -100,8 +100,8 @@ def _check(gpu, B, H, Sq, Sk, causal, seed, ref_device="cpu", autograd=True, sca
         (1, 2, 77, 130, True),      # Sq < Sk: bottom-right aligned causal
         (1, 2, 150, 70, True),      # Sq > Sk: the first rows see no key and get no gradient
         (2, 2, 96, 96, False),      # non-causal
-        (1, 2, 100, 1100, False),   # two 1024-key weight-gradient chunks
-        (1, 1, 1030, 1030, True),   # causal across the chunk boundary
+        (1, 2, 100, 1100, False),   # nine 128-key weight-gradient chunks
+        (1, 1, 1030, 1030, True),   # causal, the last chunk with six keys
         (1, 3, 5, 5, True),         # a handful of tokens
     ],
 )
@@ -283,3 +283,22 @@ def test_otf_bwd_smaller_workspace(gpu, B, H, Sq, Sk):
             assert torch.equal(a, b), name
         for name, a, b in zip(NAMES[3:], out[3:], ref[3:]):
             assert (a - b).abs().max().item() <= 1e-3, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "B,H,Sq,Sk,causal,chunk",
+    [
+        (8, 32, 5, 1100, False, 1024),    # two chunks, the last one a whole 64-key block and 12 keys
+        (8, 32, 3, 1024, True, 1024),     # one whole chunk
+        (2, 32, 5, 1700, False, 512),     # four chunks, the last one ragged
+        (2, 32, 9, 1100, True, 256),      # five chunks, the last one ragged
+        (1, 32, 40, 777, True, 128),      # seven chunks, the last one with nine keys
+    ],
+)
+def test_otf_bwd_weight_gradient_chunks(gpu, B, H, Sq, Sk, causal, chunk):
+    """Every chunk length of the weight-gradient kernel, its serial loop over 64-key blocks up to a
+    ragged end, in fp32 and with the 16-byte bf16 dK / dV stores (the default dtypes, compared bit
+    for bit with the rounded fp32 ones)."""
+    assert _wgrad_chunk(gpu, B, H, Sk) == chunk
+    _check(gpu, B, H, Sq, Sk, causal, seed=Sk + chunk, ref_device="gpu", autograd=False)
