@@ -63,7 +63,6 @@ constexpr int kPageOffset = kFlagOffset + 2 * kWaves * 4;
 // the first key tile meanwhile; the region reaches 1 KB into partial-score buffer 0, which is
 // first written after Q has been read out.
 constexpr int kQRowBytes = kDqk * 2 + 16;
-constexpr int kQChunks = kRowsPerWG * kQRowBytes / 16;   // 4672 16-byte chunks, 73 per row
 constexpr int kQOffset = kTileBytes;
 static_assert(kQOffset + kRowsPerWG * kQRowBytes <= kXOffset + kXBytes, "Q staging fits before buffer 1");
 constexpr int kLdsBytes = kPageOffset;
@@ -113,7 +112,7 @@ struct MqaParams {
   int round_ranges;    // ranges that run at once (decode_round)
   const int32_t* plan; // decode plan (see decode_plan_kernel); unused when plan_inline
   int plan_inline;     // every workgroup builds the plan in LDS (B <= kInlinePlanB, R <= kInlinePlanR)
-  int32_t* plan_out;   // with plan_inline: workgroup 0 stores the plan here (the combine reads it)
+  int32_t* plan_out;   // with plan_inline: one workgroup stores the plan here (the combine reads it)
   bf16* part_o;        // [slots, H, 512] normalised partial outputs, rounded to bf16
   float* part_lse;     // [slots, H]
   // prefill with split key ranges (PrefillSplit)
@@ -216,9 +215,10 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
       return wk.ctx - 1;
     }
   };
-  // Rows past the last one (the tail of the last item) compute the item's first row again: its
-  // Q, its limit (the smallest of the item), output discarded; so no tile below that limit needs
-  // a mask for any row of the item.
+  // Rows past the last one (the tail of the last item) have the limit of the item's first row (the
+  // smallest of the item), so no tile below that limit needs a mask for any row of the item.  Their Q is
+  // that row's too, or, in 16-row blocks that hold no row at all, row l16 of block 0's (stage_q);
+  // their output is discarded.
   const int own_lim = limit_of(own_row < nrows ? own_row : row0);
   // First tile holding a key past some row's limit (the item's first row has the smallest).
   const int first_mask_tile = max(limit_of(row0) + 1, 0) / kTileN;
@@ -851,7 +851,7 @@ struct RangeSpan {
 // ballot, and wave 0 leaves the per-sequence values in LDS.  One barrier.  The general builder below,
 // with its scans through LDS, 64-bit divisions and one thread placing all ranges of its sequence,
 // took 6.3 us of the 15.6 us the kernel ran at one sequence of 5000 tokens; with this one the call went
-// from 28.0 to 23.5 us there, and from 113.1 to 111.1 us at 64 sequences x 128 heads.  The last
+// from 28.2 to 23.7 us there, and from 110.4 to 109.2 us at 64 sequences x 128 heads.  The last
 // workgroup (whose range is the last, never longer than the others) stores the plan for the combine.
 __device__ __forceinline__ RangeSpan build_small_plan(const MqaParams& p, DMLA_LDS InlinePlan* ip, int r) {
   const int lane = fresh_lane_id();

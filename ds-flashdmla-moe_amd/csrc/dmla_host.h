@@ -25,8 +25,7 @@ int device_cu_count();
 // Split-KV combine (dmla_cache.hip): part_o [.., split, .., d] fp32 partial outputs, each
 // normalised over its split, and part_lse natural-log sums, addressed by element strides.
 // The split count of sequence b is num_splits[b] (at most max_splits) when given, else max_splits.
-// Split s of
-// sequence b is at b * sb + s * ss, or at (split_base[b] + s) * ss when split_base is given.
+// Split s of sequence b is at b * sb + s * ss, or at (split_base[b] + s) * ss when split_base is given.
 // skip_single leaves sequences with one split untouched (their rows were written by the
 // producer directly).
 // part_o16, when set, replaces part_o with bf16 partials of the same layout (the decode's own).
