@@ -695,8 +695,9 @@ __device__ __forceinline__ void mqa_fwd_body(const MqaParams& p, const MqaParams
   if (kh == 0 && g == 0 && own_row < nrows) {
     if constexpr (!kDecode) {
       if (kSplit && wk.nsplit > 1) {
+        // Keys that are all NaN have no finite score, but their sum makes the row's sum NaN.
         p.part_ml[(int64_t)wk.slot * kRowsPerWG + 16 * rb + l16] =
-            make_float2(mt, mt == kNegInf ? 0.f : ltot * fast_exp2(mref - mt));
+            make_float2(mt, mt == kNegInf ? 0.f * ltot : ltot * fast_exp2(mref - mt));
       } else if (p.m != nullptr) {
         const int pos = fast_div(own_row, p.hdiv), head = own_row - pos * p.H;
         const int si = (b * p.H + head) * p.Sq + pos;

@@ -159,3 +159,35 @@ def test_fwd_without_memory_for_the_workspace(gpu, monkeypatch):
     out = ops.flash_dmla_fwd(q, k, 512, SCALE, True)
     for a, b in zip(out, ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["one key", "a part's keys", "all keys", "a query row", "an infinite key"])
+def test_fwd_split_propagates_nan_as_unsplit(gpu, where):
+    """NaN and infinite inputs give NaN in the same places of o, m and l with and without split key
+    ranges: a part whose keys are all NaN has no finite score, but its NaN row sum still counts."""
+    B, H, Sq, Sk = 1, 16, 4, 4100      # one row tile of 129 key tiles
+    parts = ops._lib.lib().dmla_fwd_workspace_bytes(B, H, Sq, Sk, 576, 512, 1) // (64 * (512 * 4 + 8))
+    assert parts > 2
+    q = seeded((B, H, Sq, 576), 95, 0.5, torch.bfloat16).to(gpu)
+    k = seeded((B, Sk, 576), 96, 0.5, torch.bfloat16).to(gpu)
+    if where == "one key":
+        k[0, 700] = float("nan")
+    elif where == "a part's keys":
+        k[0, 129 // parts * 32:129 * 2 // parts * 32] = float("nan")
+    elif where == "all keys":
+        k[:] = float("nan")
+    elif where == "a query row":
+        q[0, 3, 2] = float("nan")
+    else:
+        k[0, 2000, :64] = float("inf")
+    plain = [torch.empty(*s, dtype=t, device=gpu) for s, t in
+             (((B, H, Sq, 512), torch.bfloat16), ((B, H, Sq), torch.float32), ((B, H, Sq), torch.float32))]
+    ops._lib.call("dmla_fwd_cache_latent", *map(ops._ptr, (q, k, *plain)), B, H, Sq, Sk, 576, 512, *q.stride()[:3],
+                  *k.stride()[:2], *plain[0].stride()[:3], SCALE, 1, ops._stream(q))
+    for name, a, b in zip(("o", "m", "l"), ops.flash_dmla_fwd(q, k, 512, SCALE, True), plain):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)), name
+        fin = torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), fin), name
+        assert (a[fin].float() - b[fin].float()).abs().max().item() <= 1e-2 * b[fin].abs().max().item() if fin.any() else True
+    assert bool(torch.isnan(plain[0]).any())
