@@ -104,3 +104,29 @@ def test_ops_launch_on_the_current_stream(gpu):
     torch.cuda.synchronize()
     assert bool(torch.isfinite(o_s).all()) and bool(torch.isfinite(lse_s).all())
     assert torch.equal(o_s, o_ref) and torch.equal(lse_s, lse_ref)
+
+
+@pytest.mark.gpu
+def test_split_prefill_and_short_onthefly_forward_replay_in_a_graph(gpu):
+    # A prefill with split key ranges (its workspace comes from the graph's pool) and the on-the-fly
+    # forward of a short sequence.
+    q = seeded((1, 16, 64, 576), 75, 0.5, torch.bfloat16).to(gpu)
+    k = seeded((1, 2000, 576), 76, 0.5, torch.bfloat16).to(gpu)
+    assert ops._lib.lib().dmla_fwd_workspace_bytes(1, 16, 64, 2000, 576, 512, 1) > 0
+    qo = seeded((1, 4, 500, 64), 77, 1.0, torch.bfloat16).to(gpu)
+    ko = seeded((1, 500, 4, 128), 78, 1.0, torch.bfloat16).to(gpu)
+    w = seeded((4, 128, 64), 79, 0.1, torch.bfloat16).to(gpu)
+
+    def step():
+        return ops.flash_dmla_fwd(q, k, 512, SCALE, True) + (ops.flash_dmla_fwd_onthefly(qo, ko, ko, w, w, 0.125, True),)
+
+    graph, outs_g = _capture(step)
+    for r in range(3):
+        q.copy_(seeded(tuple(q.shape), 500 + r, 0.5, torch.bfloat16).to(gpu))
+        qo.copy_(seeded(tuple(qo.shape), 600 + r, 1.0, torch.bfloat16).to(gpu))
+        graph.replay()
+        torch.cuda.synchronize()
+        outs_e = step()
+        torch.cuda.synchronize()
+        for name, g, e in zip(("o", "m", "l", "o (on the fly)"), outs_g, outs_e):
+            assert torch.equal(g, e), f"replay {r}: {name} differs from the eager call"
